@@ -666,14 +666,9 @@ int32_t parse_jobs(const double *jobs, int32_t count, int32_t stride, std::vecto
 // 421-424)
 int32_t ready_acts(hq::Kind k, char *xq, char *xs, const char *x, int32_t n, int32_t tokens, int64_t frame,
                    int64_t x_stride, hipStream_t s) {
-  const int32_t bias = relaxed(k) ? 64 : 0;
-  if (int32_t st = hip_status(hq::launch_quantize_x(xq, xs, x, n, bias, tokens, frame, x_stride, s), "quantize_x"))
-    return st;
-  if (ternary(k))
-    if (int32_t st = hip_status(hq::launch_interleave(xq, xs, n, tokens, frame, s), "interleave")) return st;
-  if (hq::blocks_kind(k))
-    if (int32_t st = hip_status(hq::launch_sums_x(xs, xq, n, tokens, frame, s), "sums_x")) return st;
-  return HQ_OK;
+  // (check_job: xq 16-byte aligned; matmuls_alike: x and x_stride too)
+  const hq::Ready mode = ternary(k) ? hq::kReadyPlanes : hq::blocks_kind(k) ? hq::kReadySums : hq::kReadyBytes;
+  return hip_status(hq::launch_ready(mode, xq, xs, x, n, relaxed(k) ? 64 : 0, tokens, frame, x_stride, s), "quantize_x");
 }
 
 // matmulsAlike (src/runtime/forward/engine.ts:398-407): a kind at a time, the input readied as that kind's jobs take

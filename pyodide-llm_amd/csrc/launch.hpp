@@ -36,6 +36,11 @@ constexpr int32_t kSbCodebooks = 33808;  // the bytes of the codebooks row it is
 // activations: count tokens of n values (x + t x_stride) -> xq + t frame, xs + t frame
 hipError_t launch_quantize_x(char *xq, char *xs, const char *x, int32_t n, int32_t bias, int32_t count,
                              int64_t frame, int64_t x_stride, hipStream_t s);
+// the same with interleave()'s planes and sums (kReadyPlanes) or sums_x's sums (kReadySums) in the one launch: x and
+// x_stride 16-byte aligned, xq 4-byte aligned; kReadyBytes: quantize_x alone
+enum Ready { kReadyBytes, kReadyPlanes, kReadySums };
+hipError_t launch_ready(Ready mode, char *xq, char *xs, const char *x, int32_t n, int32_t bias, int32_t count,
+                        int64_t frame, int64_t x_stride, hipStream_t s);
 hipError_t launch_interleave(char *xq, char *xs, int32_t n, int32_t count, int64_t frame, hipStream_t s);
 hipError_t launch_int8_sums(int32_t *out, const char *w, int32_t groups, hipStream_t s);
 hipError_t launch_six_sums(int32_t *out, const char *w, int32_t groups, hipStream_t s);

@@ -1,0 +1,88 @@
+"""The activations readied in one launch: quantize_x's bytes and scales with interleave's planes and sums (ternary) or
+sums_x's sums (llama.cpp's blocks), as hq_matmuls leaves them in the jobs' a / b, byte for byte against the oracle, at
+widths that end inside a block of 1024 values; and quantize_x where its addresses do not take 16-byte loads."""
+import numpy as np
+import pytest
+
+from gpu_util import Arena, same_bits
+from models import F
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def arena():
+    return Arena(1 << 27)
+
+
+@pytest.fixture(autouse=True)
+def fresh(arena):
+    arena.reset()
+    yield
+
+
+def activations(rng, tokens, n):
+    """groups of every size, and one each of zeros, -0, an infinity, a NaN in groupMax's lane 0 and in another, and
+    subnormals"""
+    x = (rng.standard_normal((tokens, n)) * np.exp(rng.uniform(-8, 8, (tokens, n // 32, 1))).repeat(32, 1).reshape(
+        tokens, n)).astype(F)
+    x[0, :32] = 0.0
+    x[0, 5] = -0.0
+    x[-1, 32 + 6] = np.inf
+    x[-1, 64 + 4] = np.nan
+    x[0, 96 + 7] = np.nan
+    x[0, 97] = 2.0 ** -140
+    return x
+
+
+@pytest.mark.parametrize("kind,n", [("matmul_t2r", 128), ("matmul_t2r", 1152), ("matmul_t2r", 17408),
+                                    ("matmul_sbr", 256), ("matmul_sbr", 1280), ("matmul_q8r", 128),
+                                    ("matmul_q8r", 1056)])
+@pytest.mark.parametrize("tokens", [1, 3])
+def test_readied_in_one_launch(pkg, arena, oracle, kind, n, tokens):
+    from pyodide_llm_amd import jobs
+    rng = np.random.default_rng(n + tokens)
+    x = activations(rng, tokens, n)
+    frame = 2 * n + 64
+    acts = arena.alloc(tokens * frame, fill=np.full(tokens * frame, 0xAA, np.uint8))
+    w = arena.put(np.zeros(4 * n, np.uint8))  # a row of any packing, and its scales or tables
+    out = arena.alloc(4 * tokens)
+    table = [jobs.job(kind, out, acts, acts + n, w, arena.put(np.zeros(40000, np.uint8)),
+                      12 if kind == "matmul_sbr" else 0, n, rows=1, count=tokens, os=4, as_=frame, bs=frame)]
+    L = pkg.library()
+    assert jobs.matmuls(L, arena.put(x), 4 * n, table) == 0, L.hq_last_error_message()
+    got = arena.get(acts, np.uint8, tokens * frame).reshape(tokens, frame)
+    for t in range(tokens):
+        q, scales = oracle.quantize_x(x[t], 64 if kind == "matmul_q8r" else 0)
+        area = scales
+        if kind == "matmul_t2r":
+            q, area = oracle.interleave(q.view(np.int8), scales)
+        elif kind == "matmul_sbr":
+            area = oracle.sums_x(q.view(np.int8), scales)
+        want = np.full(frame, 0xAA, np.uint8)
+        bytes_ = np.ascontiguousarray(area).view(np.uint8)
+        want[:n] = q.view(np.uint8)
+        want[n:n + bytes_.size] = bytes_
+        # (a NaN's own bits are not compared)
+        mine, theirs = got[t].copy(), want
+        for row in (mine, theirs):
+            s = row[n:n + n // 8].view(F)
+            s[np.isnan(s)] = np.nan
+        assert np.array_equal(mine, theirs), (t, np.nonzero(mine != theirs)[0][:8])
+
+
+@pytest.mark.parametrize("x_off,xq_off", [(4, 0), (0, 1), (8, 2), (0, 4)])
+def test_quantize_x_anywhere(pkg, arena, oracle, x_off, xq_off):
+    rng = np.random.default_rng(x_off + 16 * xq_off)
+    n = 1056
+    x = rng.standard_normal(n).astype(F)
+    ax = arena.alloc(4 * n + 16) + x_off
+    arena.write(ax, x)
+    xq = arena.alloc(n + 16, fill=np.full(n + 16, 0xAA, np.uint8)) + xq_off
+    xs = arena.alloc(4 * (n // 32))
+    assert pkg.library().hq_quantize_x_ex(xq, xs, ax, n, 64, None) == 0
+    want_q, want_s = oracle.quantize_x(x, 64)
+    got = arena.get(xq - xq_off, np.uint8, n + 16)
+    assert np.array_equal(got[xq_off:xq_off + n], want_q)
+    assert np.all(got[:xq_off] == 0xAA) and np.all(got[xq_off + n:] == 0xAA)
+    assert same_bits(arena.get(xs, F, n // 32), want_s)

@@ -285,7 +285,8 @@ int32_t hq_tol_min_tiles(int32_t tiles);
 /* Which kernels take a job of `kind` (hq_phase's numbers), row length n and `count` tokens whose activations are
  * frame bytes apart and their scales sframe: 1 the matrix-core tile (16 tokens or more, and every offset within a
  * tile of 64 tokens, 128 for llama.cpp's blocks, and of 128 rows below 4 GiB), 0 the token kernel (4 tokens a
- * launch: the same numbers), -1 a kind not run here.  Host-only: no device is touched. */
+ * launch: the same numbers), -1 a kind not run here.  (The counts between, about 5 to 64 tokens, run on the matrix
+ * cores' few-token tiles whichever of the two this says: the same numbers.)  Host-only: no device is touched. */
 int32_t hq_job_path(int32_t kind, int32_t n, int32_t count, int64_t frame, int64_t sframe);
 
 /* The ceilings the kernels are measured against (no counterpart on this path: the reference's CPU ceiling loops,

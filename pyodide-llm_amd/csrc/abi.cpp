@@ -23,8 +23,17 @@ std::atomic<void *> g_stream{nullptr};
 // hq_tol_min_tiles's setting: -1, one round of two blocks a compute unit
 std::atomic<int32_t> g_tol_min_tiles{-1};
 
-// more tokens than this take the matrix cores (fewer: the token kernel, the weights read once a 4 tokens)
+// as many tokens or more take the prompt tiles, where few.hip (few_tokens) does not take them first; fewer the token
+// kernel, the weights read once a 4 tokens
 constexpr int32_t kGemmMinTokens = 16;
+
+// whether a tile's offsets fit in 32 bits
+bool tile_offsets_fit(hq::Kind kind, const hq::Job &j) {
+  constexpr int64_t kLimit = (int64_t)1 << 32;
+  const int64_t row_bytes = hq::signs_kind(kind) ? (int64_t)(j.n >> 7) * 32 : (int64_t)(j.n >> 5) * 32;
+  const int64_t scales = hq::signs_kind(kind) ? 8 * (int64_t)(j.n >> 5) : 4 * (int64_t)(j.n >> 5);
+  return 64 * j.frame + j.n < kLimit && 64 * j.sframe + scales < kLimit && 128 * row_bytes < kLimit;
+}
 
 // Which kernels take a job: 1 the matrix-core tile, 0 the token kernel (4 tokens a launch).  The tiles keep a lane's
 // offsets within a tile in 32 bits: 64 tokens of activations (frame and sframe bytes apart: 128 for the blocks' tile)
@@ -35,11 +44,19 @@ int32_t path_of(hq::Kind kind, const hq::Job &j) {
     return j.count >= hq::kSbTileMin && j.frame > 0 && j.sframe > 0 && j.frame < hq::kSbTileFrameMax &&
            j.sframe < hq::kSbTileFrameMax;
   }
-  if (j.count < kGemmMinTokens || !hq::gemm_supported(kind)) return 0;
-  constexpr int64_t kLimit = (int64_t)1 << 32;
-  const int64_t row_bytes = hq::signs_kind(kind) ? (int64_t)(j.n >> 7) * 32 : (int64_t)(j.n >> 5) * 32;
-  const int64_t scales = hq::signs_kind(kind) ? 8 * (int64_t)(j.n >> 5) : 4 * (int64_t)(j.n >> 5);
-  return 64 * j.frame + j.n < kLimit && 64 * j.sframe + scales < kLimit && 128 * row_bytes < kLimit;
+  return j.count >= kGemmMinTokens && hq::gemm_supported(kind) && tile_offsets_fit(kind, j);
+}
+
+// The jobs that few.hip's 16-token tiles take: from the token counts where its one pass over the weights beats the token
+// kernel's pass a 4 tokens, to those where gemm.hip's larger tiles fill the GPU.  Measured both ways (us, token kernel or
+// prompt tile / few.hip): an 8B layer of int8 at 4 tokens 65 / 76, 5 tokens 109 / 76, 64 tokens 214 / 168, 80 tokens
+// 200 / 206; the 27B MLP of int6 at 4 tokens 70 / 90, 64 tokens 225 / 212, of ternary at 2 tokens 37 / 66, 3 tokens 72 /
+// 67, 160 tokens 342 / 318, 192 tokens 347 / 356.
+constexpr int32_t kFewMin = 5, kFewMax = 64, kFewSignsMin = 3, kFewSignsMax = 160;
+bool few_tokens(hq::Kind kind, const hq::Job &j) {
+  const bool signs = hq::signs_kind(kind);
+  return hq::gemm_supported(kind) && j.count >= (signs ? kFewSignsMin : kFewMin) &&
+         j.count <= (signs ? kFewSignsMax : kFewMax) && tile_offsets_fit(kind, j);
 }
 
 int32_t fail(int32_t code, const char *fmt, ...) {
@@ -188,7 +205,7 @@ int32_t check_job(hq::Kind kind, const hq::Job &j, int32_t three) {
   return HQ_OK;
 }
 
-// runs jobs of one kind: GEMV jobs (up to 4 tokens; more in slices of 4) batched in launches of up to kMaxJobs,
+// runs jobs of one kind: few-token jobs and GEMV jobs (up to 4 tokens; more in slices of 4) batched in launches of up to kMaxJobs,
 // GEMM jobs one a launch
 int32_t run_blocks(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s) {
   // up to 4 tokens a launch (a prompt in slices of 4: every (row, token) the token kernel's number), jobs of one
@@ -229,8 +246,13 @@ int32_t run_blocks(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t 
 int32_t run_jobs(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s) {
   if (hq::blocks_kind(kind)) return run_blocks(kind, jobs, s);
   std::vector<hq::Job> gemv[hq::kGemvMaxTokens + 1][2];  // by token count, by wc-ness
+  std::vector<hq::Job> few;
   for (const hq::Job &j : jobs) {
     if (j.r1 == j.r0 || j.count == 0) continue;
+    if (few_tokens(kind, j)) {
+      few.push_back(j);
+      continue;
+    }
     if (path_of(kind, j)) {
       const int32_t st = hip_status(hq::launch_gemm(kind, j, s), kind_name(kind));
       if (st) return st;
@@ -244,6 +266,21 @@ int32_t run_jobs(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s)
       part.xs = j.xs + t0 * j.sframe;
       gemv[part.count][part.wc != nullptr].push_back(part);
     }
+  }
+  for (size_t i = 0; i < few.size();) {  // a launch: jobs of one token count, all with wc or none
+    hq::Job same[hq::kMaxJobs];
+    int32_t m = 0;
+    size_t kept = i;
+    const int32_t count = few[i].count;
+    const bool wc = few[i].wc != nullptr;
+    for (size_t e = i; e < few.size(); e++) {
+      if (m < hq::kMaxJobs && few[e].count == count && (few[e].wc != nullptr) == wc) {
+        same[m++] = few[e];
+        std::swap(few[e], few[kept++]);
+      }
+    }
+    i = kept;
+    if (int32_t st = hip_status(hq::launch_few(kind, same, m, s), kind_name(kind))) return st;
   }
   for (int c = 1; c <= hq::kGemvMaxTokens; c++)
     for (int w = 0; w < 2; w++) {

@@ -101,6 +101,10 @@ hipError_t launch_take_channels(float *picked, float *x, const Channels &ch, hip
 // matmul_t2r_tile over a prompt.  Returns hipErrorNotSupported for a kind that has none.
 hipError_t launch_gemm(Kind kind, const Job &job, hipStream_t s);
 
+// a few tokens on the matrix cores (few.hip): jobs of one kind (as launch_gemm's), one token count and all with wc or
+// none, up to kMaxJobs a launch
+hipError_t launch_few(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s);
+
 // the relaxed int8 prompt tile to float32 tolerance (gemm_tol.hip): the job's activations widened into `work`
 // (tol_work_bytes(n, count) bytes, 256-byte aligned), then the tiles; job.wc is not read (corrections derived)
 int64_t tol_work_bytes(int32_t n, int32_t count);

@@ -20,10 +20,11 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 OBJ = os.path.join(HERE, "_build")
 LIBRARY = os.path.join(HERE, "libhq.so")
-SOURCES = ["quantize.hip", "gemv.hip", "gemm.hip", "gemm_tol.hip", "few.hip", "blocks.hip", "columns.hip", "ceilings.hip", "abi.cpp"]
+SOURCES = ["quantize.hip", "gemv.hip", "gemm.hip", "gemm_tol.hip", "few.hip", "blocks.hip", "q4k.hip", "columns.hip", "ceilings.hip", "abi.cpp"]
 # blocks.hip's prompt tile keeps its matrix-core results in ordinary VGPRs (no copies out of AGPRs: it has registers
 # to spare and reads every result on the VALU)
 EXTRA = {"blocks.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+         "q4k.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
          # the token kernels' scalar arguments (one job's fields) in the waves' scalar registers at launch
          "gemv.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
          # quantize_x's arguments likewise (14 dwords): it runs before every phase of a decode step

@@ -205,14 +205,39 @@ int32_t check_job(hq::Kind kind, const hq::Job &j, int32_t three) {
   return HQ_OK;
 }
 
+// jobs in launches of up to kMaxJobs of one token count, all with wc or none
+template <typename Launch>
+int32_t run_together(std::vector<hq::Job> &jobs, hq::Kind kind, Launch launch) {
+  for (size_t i = 0; i < jobs.size();) {
+    hq::Job same[hq::kMaxJobs];
+    int32_t m = 0;
+    size_t kept = i;
+    const int32_t count = jobs[i].count;
+    const bool wc = jobs[i].wc != nullptr;
+    for (size_t e = i; e < jobs.size(); e++) {
+      if (m < hq::kMaxJobs && jobs[e].count == count && (jobs[e].wc != nullptr) == wc) {
+        same[m++] = jobs[e];
+        std::swap(jobs[e], jobs[kept++]);
+      }
+    }
+    i = kept;
+    if (int32_t st = hip_status(launch(same, m), kind_name(kind))) return st;
+  }
+  return HQ_OK;
+}
+
 // runs jobs of one kind: few-token jobs and GEMV jobs (up to 4 tokens; more in slices of 4) batched in launches of up to kMaxJobs,
 // GEMM jobs one a launch
 int32_t run_blocks(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s) {
   // up to 4 tokens a launch (a prompt in slices of 4: every (row, token) the token kernel's number), jobs of one
   // block type, one token count and one tables' area together
-  std::vector<hq::Job> parts;
+  std::vector<hq::Job> parts, q4k;
   for (const hq::Job &j : jobs) {
     if (j.r1 == j.r0 || j.count == 0) continue;
+    if (hq::q4k_tile(j)) {
+      q4k.push_back(j);
+      continue;
+    }
     // a prompt: the matrix-core tile (its offsets within a tile of tokens are 32-bit: frames under 16 MB)
     if (path_of(kind, j)) {
       const int32_t st = hip_status(hq::launch_sb_tile(j, s), kind_name(kind));
@@ -228,6 +253,8 @@ int32_t run_blocks(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t 
       parts.push_back(part);
     }
   }
+  if (int32_t st = run_together(q4k, kind, [&](const hq::Job *same, int32_t m) { return hq::launch_q4k(same, m, s); }))
+    return st;
   std::vector<bool> done(parts.size(), false);
   for (size_t i = 0; i < parts.size(); i++) {
     if (done[i]) continue;
@@ -267,21 +294,8 @@ int32_t run_jobs(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s)
       gemv[part.count][part.wc != nullptr].push_back(part);
     }
   }
-  for (size_t i = 0; i < few.size();) {  // a launch: jobs of one token count, all with wc or none
-    hq::Job same[hq::kMaxJobs];
-    int32_t m = 0;
-    size_t kept = i;
-    const int32_t count = few[i].count;
-    const bool wc = few[i].wc != nullptr;
-    for (size_t e = i; e < few.size(); e++) {
-      if (m < hq::kMaxJobs && few[e].count == count && (few[e].wc != nullptr) == wc) {
-        same[m++] = few[e];
-        std::swap(few[e], few[kept++]);
-      }
-    }
-    i = kept;
-    if (int32_t st = hip_status(hq::launch_few(kind, same, m, s), kind_name(kind))) return st;
-  }
+  if (int32_t st = run_together(few, kind, [&](const hq::Job *same, int32_t m) { return hq::launch_few(kind, same, m, s); }))
+    return st;
   for (int c = 1; c <= hq::kGemvMaxTokens; c++)
     for (int w = 0; w < 2; w++) {
       const auto &list = gemv[c][w];

@@ -82,6 +82,10 @@ hipError_t launch_sb(const Job *jobs, int32_t njobs, hipStream_t s);
 constexpr int kSbTileMin = 16;
 constexpr int64_t kSbTileFrameMax = (int64_t)1 << 24;  // frame and sframe of a job the tile takes: 128 tokens' offsets fit in int32
 hipError_t launch_sb_tile(const Job &job, hipStream_t s);
+// a few tokens or a prompt of Q4_K (q4k.hip): whether a job is one that its tiles take, and the launch of up to kMaxJobs such jobs
+// of one token count
+bool q4k_tile(const Job &j);
+hipError_t launch_q4k(const Job *jobs, int32_t njobs, hipStream_t s);
 hipError_t launch_signed_dots(int32_t *out, const int8_t *a, const int8_t *b, hipStream_t s);
 
 // the classifier's outlier channels: add_columns (y += the columns' products, in order); the columns of a packed

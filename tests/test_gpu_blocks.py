@@ -323,3 +323,52 @@ def test_signed_dots(k, arena):
     k.signed_dots(out, arena.put(a), arena.put(b))
     want = (a.astype(np.int32) * b.astype(np.int32)).reshape(4, 4).sum(1)
     assert np.array_equal(arena.get(out, np.int32, 4), want)
+
+
+@pytest.mark.parametrize("n,rows,tokens", [(256, 33, 3), (512, 16, 16), (1280, 50, 17), (256, 1, 32), (1024, 65, 33),
+                                           (768, 12400, 33), (512, 12300, 70)])
+def test_q4k_tiles(pkg, arena, oracle, setup, n, rows, tokens):
+    """Q4_K's own tiles (16-byte aligned blocks, three tokens or more): 16 x 16 tiles and, for launches of many tiles,
+    32 x 32 ones, cut inside a tile, two jobs of one input in a launch, a row range inside the matrix, nothing else
+    written; and blocks 2 bytes into a word (the general tile or token kernel), the same numbers"""
+    from pyodide_llm_amd import jobs
+    row, tab = setup
+    area = arena.alloc(34992)
+    L = pkg.library()
+    assert L.hq_sb_tables_ex(area, arena.put(row), None) == 0
+    rng = np.random.default_rng(n + rows + tokens)
+    frame = 2 * n
+    buf = np.zeros((tokens, frame), np.uint8)
+    ready = []
+    for t in range(tokens):
+        q, area_t = token_area(oracle, rng, n, 1.0 + t)
+        buf[t, :n], buf[t, n:n + area_t.size] = q.view(np.uint8), area_t.view(np.uint8)
+        ready.append((q, area_t))
+    a = arena.put(buf)
+    mats = [bm.random_blocks(rng, 12, r * (n // 256)) for r in (rows, 19)]
+    sample = sorted(set(rng.integers(0, tokens, 4)) | {0, tokens - 1})
+    for shift in (0, 2):
+        table, outs = [], []
+        for blocks in mats:
+            r = len(blocks) // (n // 256)
+            w = arena.alloc(blocks.size + 16) + shift
+            arena.write(w, blocks)
+            os = 4 * r + 8
+            out = arena.alloc(tokens * os, fill=np.full(tokens * os // 4, -7, F))
+            table.append(jobs.job("matmul_sbr", out, a, a + n, w, area, 12, n, rows=r, count=tokens, os=os, as_=frame,
+                                  bs=frame))
+            outs.append((out, os, r, blocks))
+        assert jobs.phase(L, table) == 0, L.hq_last_error_message()
+        for out, os, r, blocks in outs:
+            got = arena.get(out, F, tokens * os // 4).reshape(tokens, os // 4)
+            assert np.all(got[:, r:] == -7)
+            for t in sample:
+                want = oracle.matmul_sbr(*ready[t], blocks, tab, n, 12)
+                assert same_bits(got[t, :r], want), (shift, t, first_difference(got[t, :r], want))
+    if rows > 20:
+        out = arena.alloc(4 * tokens * rows, fill=np.full(tokens * rows, -7, F))
+        w = arena.put(mats[0])
+        assert L.hq_matmul_sbr_tile_ex(out, a, a + n, w, area, n, 5, rows - 3, tokens, 4 * rows, frame, 12, None) == 0
+        got = arena.get(out, F, tokens * rows).reshape(tokens, rows)
+        want = oracle.matmul_sbr(*ready[-1], mats[0], tab, n, 12)
+        assert np.all(got[:, :5] == -7) and np.all(got[:, rows - 3:] == -7) and same_bits(got[-1, 5:rows - 3], want[5:rows - 3])

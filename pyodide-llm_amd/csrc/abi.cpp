@@ -722,6 +722,21 @@ int32_t ready_acts(hq::Kind k, char *xq, char *xs, const char *x, int32_t n, int
   return hip_status(hq::launch_ready(mode, xq, xs, x, n, relaxed(k) ? 64 : 0, tokens, frame, x_stride, s), "quantize_x");
 }
 
+bool overlap(const char *a, int64_t an, const char *b, int64_t bn) { return a < b + bn && b < a + an; }
+
+// One token's jobs of a kind run from the float32 input itself, their readied activations written by the way: where the
+// kernels do so (gemv_ready_takes, sb_ready_takes), every job has one a / b, and the input, which every block of the
+// launch reads, overlaps nothing the launch writes.
+bool ready_in_launch(hq::Kind k, const std::vector<hq::Job> &list, const char *x) {
+  const hq::Job &first = list[0];
+  if (first.count != 1 || list.size() > (size_t)hq::kMaxJobs) return false;
+  for (const hq::Job &j : list)
+    if (j.xq != first.xq || j.xs != first.xs || overlap(x, 4 * (int64_t)j.n, j.out, 4 * (int64_t)j.r1)) return false;
+  if (overlap(x, 4 * (int64_t)first.n, first.xq, first.n) || overlap(x, 4 * (int64_t)first.n, first.xs, first.n / 2)) return false;
+  return hq::blocks_kind(k) ? hq::sb_ready_takes(list.data(), (int32_t)list.size())
+                            : hq::gemv_ready_takes(k, list.data(), (int32_t)list.size());
+}
+
 // matmulsAlike (src/runtime/forward/engine.ts:398-407): a kind at a time, the input readied as that kind's jobs take
 // it, then those jobs run as hq_phase runs them.  staging NULL: into the jobs' own a / b (a pair several jobs share
 // readied once); else into staging (every job's a / b replaced by it, its tokens `frame` bytes apart), kind after
@@ -759,19 +774,21 @@ int32_t matmuls_alike(const void *x, int32_t x_stride, std::vector<hq::Job> by_k
     auto &list = by_kind[kind];
     if (list.empty()) continue;
     const hq::Kind k = (hq::Kind)kind;
-    if (staging) {
-      if (int32_t st = ready_acts(k, staging, staging + qbytes, (const char *)x, n, tokens, frame, x_stride, s))
-        return st;
+    if (staging)
       for (hq::Job &j : list) j.xq = staging, j.xs = staging + qbytes, j.frame = frame, j.sframe = frame;
-    } else {
-      for (size_t i = 0; i < list.size(); i++) {
-        const hq::Job &j = list[i];
-        bool seen = false;
-        for (size_t e = 0; e < i && !seen; e++) seen = list[e].xq == j.xq && list[e].xs == j.xs && list[e].frame == j.frame;
-        if (seen) continue;
-        if (int32_t st = ready_acts(k, (char *)j.xq, (char *)j.xs, (const char *)x, n, tokens, j.frame, x_stride, s))
-          return st;
-      }
+    if (ready_in_launch(k, list, (const char *)x)) {
+      const hipError_t e = hq::blocks_kind(k) ? hq::launch_sb_ready((const char *)x, list.data(), (int32_t)list.size(), s)
+                                              : hq::launch_gemv_ready(k, (const char *)x, list.data(), (int32_t)list.size(), s);
+      if (int32_t st = hip_status(e, kind_name(k))) return st;
+      continue;
+    }
+    for (size_t i = 0; i < list.size(); i++) {
+      const hq::Job &j = list[i];
+      bool seen = false;
+      for (size_t e = 0; e < i && !seen; e++) seen = list[e].xq == j.xq && list[e].xs == j.xs && list[e].frame == j.frame;
+      if (seen) continue;
+      if (int32_t st = ready_acts(k, (char *)j.xq, (char *)j.xs, (const char *)x, n, tokens, j.frame, x_stride, s))
+        return st;
     }
     if (int32_t st = run_jobs(k, list, s)) return st;
   }

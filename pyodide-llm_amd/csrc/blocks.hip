@@ -226,6 +226,7 @@ HQ_DEV float block_fm(const BB &B) {
 // and its waves take units (a wave's 64 / L rows) in turn.
 // ---------------------------------------------------------------------------------------------------------------
 struct SbBatch {
+  const char *x;  // READY: the token's float32 input
   Job job[kMaxJobs];
   int32_t unit0[kMaxJobs + 1];  // the first group of 4 rows of each job; unit0[njobs]: the groups of the launch
   int32_t njobs;
@@ -373,7 +374,10 @@ template <int TY> constexpr int lds_table_bytes() {
 // (one token: 16 against 4, 3-10 % faster for every type); 2..4 tokens keep 4 (their registers: 16 waves a block
 // leave a wave 128)
 template <int T> constexpr int sb_waves() { return T == 1 ? 16 : 4; }
-template <int TY, int T, int L, bool STAGE, bool COAL>
+// READY (STAGE): the block makes its staged copy from the float32 input itself (a block has 1024 threads, so 4096 values are
+// one round of theirs), the first block writing the caller's xq and xs too, instead of a launch of ready_kernel before
+// (the 8B gate/up and down of a token, us: Q4_K 31.0 -> 29.9; a 1024-wide model's 18.5 -> 15.4).
+template <int TY, int T, int L, bool STAGE, bool COAL, bool READY>
 __global__ __launch_bounds__(64 * sb_waves<T>()) void gemv_sb(SbBatch batch) {
   constexpr int kSbWaves = sb_waves<T>();
   constexpr int R = 64 / L;  // rows a wave
@@ -391,7 +395,32 @@ __global__ __launch_bounds__(64 * sb_waves<T>()) void gemv_sb(SbBatch batch) {
       for (int i = threadIdx.x; i < 1024 / 16; i += 64 * kSbWaves)
         ((uint4 *)(table + GRID))[i] = ((const uint4 *)(tab + T_SIGNS))[i];
   }
-  if (STAGE) {
+  if (READY) {
+    const Job &J0 = batch.job[0];
+    const int n = J0.n, acts = (n >> 8) * kSbPitch, tid = threadIdx.x;
+    const bool keep = blockIdx.x == 0;
+    float *xs = (float *)J0.xs;
+    int16_t *s16 = (int16_t *)(xs + (n >> 5)), *s8 = s16 + (n >> 4);
+    for (int first = 0; first < n; first += 4 * 64 * kSbWaves) {
+      const int at = first + 4 * tid;
+      const bool live = at < n;
+      const Quantized4 o = quantize4(*(const float4 *)(batch.x + 4 * (int64_t)(live ? at : 0)), 0);
+      if (!live) continue;
+      char *blk = staged + (at >> 8) * (stages_sums<TY>() ? kSbPitchSums : kSbPitch);
+      *(uint32_t *)(blk + (at & 255)) = o.d;
+      if ((tid & 7) == 0) *(float *)(stages_sums<TY>() ? blk + 256 + 4 * ((at >> 5) & 7) : staged + acts + 4 * (at >> 5)) = o.scale;
+      if (stages_sums<TY>()) {
+        if ((tid & 3) == 0) *(int16_t *)(blk + 288 + 2 * ((at >> 4) & 15)) = (int16_t)o.s16;
+        if ((tid & 1) == 0) *(int16_t *)(blk + 320 + 2 * ((at >> 3) & 31)) = (int16_t)o.s8;
+      }
+      if (keep) {
+        *(uint32_t *)((char *)J0.xq + at) = o.d;
+        if ((tid & 7) == 0) xs[at >> 5] = o.scale;
+        if ((tid & 3) == 0) s16[at >> 4] = (int16_t)o.s16;
+        if ((tid & 1) == 0) s8[at >> 3] = (int16_t)o.s8;
+      }
+    }
+  } else if (STAGE) {
     const Job &J0 = batch.job[0];
     const int per = J0.n + J0.n / 2, acts = (J0.n >> 8) * kSbPitch, n8 = J0.n >> 3;
     for (int i = threadIdx.x; i < per / 16; i += 64 * kSbWaves) {
@@ -541,7 +570,7 @@ __global__ __launch_bounds__(64 * sb_waves<T>()) void gemv_sb(SbBatch batch) {
 
 // a launch's blocks: as many as stay resident together (at most the units over the waves a block); lds: the staged
 // activations' bytes (0: none)
-template <int TY, int T, int L, bool STAGE, bool COAL>
+template <int TY, int T, int L, bool STAGE, bool COAL, bool READY = false>
 hipError_t launch_tt(const SbBatch &b, size_t lds, hipStream_t s) {
   static int per_cu[64][16];  // by device and 4 KB of staged bytes
   int dev = 0;
@@ -549,7 +578,7 @@ hipError_t launch_tt(const SbBatch &b, size_t lds, hipStream_t s) {
   const int slot = (int)(lds / 4096) < 16 ? (int)(lds / 4096) : 15;
   if (per_cu[dev][slot] == 0) {
     int k = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, gemv_sb<TY, T, L, STAGE, COAL>, 64 * sb_waves<T>(),
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, gemv_sb<TY, T, L, STAGE, COAL, READY>, 64 * sb_waves<T>(),
                                                      4096 * (slot + 1)) !=
             hipSuccess || k < 1)
       k = 1;
@@ -557,8 +586,15 @@ hipError_t launch_tt(const SbBatch &b, size_t lds, hipStream_t s) {
   }
   constexpr int W = sb_waves<T>();
   const int want = (b.unit0[b.njobs] + W - 1) / W, cap = per_cu[dev][slot] * cu_count();
-  hipLaunchKernelGGL((gemv_sb<TY, T, L, STAGE, COAL>), dim3(want < cap ? want : cap), dim3(64 * W), lds, s, b);
+  hipLaunchKernelGGL((gemv_sb<TY, T, L, STAGE, COAL, READY>), dim3(want < cap ? want : cap), dim3(64 * W), lds, s, b);
   return hipGetLastError();
+}
+
+// one token, its activations staged
+template <int TY, bool COAL>
+hipError_t launch_one(const SbBatch &b, int L, size_t lds, hipStream_t s) {
+  if (b.x) return L == 64 ? launch_tt<TY, 1, 64, true, COAL, true>(b, lds, s) : launch_tt<TY, 1, 16, true, COAL, true>(b, lds, s);
+  return L == 64 ? launch_tt<TY, 1, 64, true, COAL>(b, lds, s) : launch_tt<TY, 1, 16, true, COAL>(b, lds, s);
 }
 
 template <int TY>
@@ -572,10 +608,9 @@ hipError_t launch_type(const SbBatch &b, int T, int L, size_t lds, hipStream_t s
           const int64_t row_bytes = (int64_t)(b.job[j].n >> 8) * sb_block_bytes(TY);
           coal = coal && ((uintptr_t)b.job[j].wq & 15u) == 0 && row_bytes % 16 == 0;
         }
-        if (coal)
-          return L == 64 ? launch_tt<TY, 1, 64, true, true>(b, lds, s) : launch_tt<TY, 1, 16, true, true>(b, lds, s);
+        if (coal) return launch_one<TY, true>(b, L, lds, s);
       }
-      return L == 64 ? launch_tt<TY, 1, 64, true, false>(b, lds, s) : launch_tt<TY, 1, 16, true, false>(b, lds, s);
+      return launch_one<TY, false>(b, L, lds, s);
     }
     return L == 64 ? launch_tt<TY, 1, 64, false, false>(b, 0, s) : launch_tt<TY, 1, 16, false, false>(b, 0, s);
   case 2: return launch_tt<TY, 2, 16, false, false>(b, 0, s);
@@ -1154,9 +1189,22 @@ hipError_t launch_sb_tile(const Job &j, hipStream_t s) {
 }
 
 // jobs: one block type, one token count (1..4), one tables' area
-hipError_t launch_sb(const Job *jobs, int32_t njobs, hipStream_t s) {
-  if (njobs < 1 || njobs > kMaxJobs) return hipErrorInvalidValue;
+hipError_t launch_sb(const Job *jobs, int32_t njobs, hipStream_t s) { return launch_sb_ready(nullptr, jobs, njobs, s); }
+
+// whether a launch of one token's jobs stages its activations (so can make them itself: launch_sb_ready)
+bool sb_ready_takes(const Job *jobs, int32_t njobs) {
+  if (njobs < 1 || njobs > kMaxJobs) return false;
+  for (int j = 0; j < njobs; j++)
+    if (jobs[j].count != 1 || jobs[j].type != jobs[0].type || jobs[j].ws != jobs[0].ws || jobs[j].n != jobs[0].n ||
+        jobs[j].xq != jobs[0].xq || jobs[j].xs != jobs[0].xs)
+      return false;
+  return sb_stage_bytes(jobs[0].type, jobs[0].n) <= kSbStageMax;
+}
+
+hipError_t launch_sb_ready(const char *x, const Job *jobs, int32_t njobs, hipStream_t s) {
+  if (njobs < 1 || njobs > kMaxJobs || (x && !sb_ready_takes(jobs, njobs))) return hipErrorInvalidValue;
   SbBatch b{};
+  b.x = x;
   int longest = 0;
   for (int j = 0; j < njobs; j++) longest = (jobs[j].n >> 8) > longest ? (jobs[j].n >> 8) : longest;
   // (a prompt's slices of 2..4 tokens keep 16 lanes: their steps are long enough)

@@ -72,6 +72,51 @@ HQ_DEV int32_t trunc_sat(float v) {
   return (int32_t)v;
 }
 
+// v_perm_b32: byte i of the result is byte sel.i of {hi:lo} (0..3 from lo, 4..7 from hi)
+HQ_DEV uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) { return __builtin_amdgcn_perm(hi, lo, sel); }
+
+// quantize_x (kernels/kernel/quantize.ts:124-151) of 4 consecutive values a lane, 8 lanes a group of 32 (every lane of a
+// group live): the lane's 4 bytes, the group's scale, and the sums of the lane's 4, its 8 and its 16 values' bytes.
+// Value 4 i + r of a group is component r of its lane i, so a component's largest |value| over the 8 lanes is groupMax's
+// lane r (a non-negative float's bits order as the float does, and every NaN's are above +inf's); lanes 1..3 are then
+// compared with lane 0's in order, where a NaN is passed over (quantize.ts:10-19).
+struct Quantized4 {
+  uint32_t d;
+  float scale;
+  int32_t s4, s8, s16;
+};
+HQ_DEV uint32_t max8(uint32_t m) {
+  m = max(m, (uint32_t)dpp<0xB1>((int32_t)m));   // quad_perm [1, 0, 3, 2]
+  m = max(m, (uint32_t)dpp<0x4E>((int32_t)m));   // quad_perm [2, 3, 0, 1]
+  return max(m, (uint32_t)dpp<0x141>((int32_t)m));  // row_half_mirror
+}
+HQ_DEV Quantized4 quantize4(const float4 &f, int32_t bias) {
+  const float v[4] = {f.x, f.y, f.z, f.w};
+  uint32_t m[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) m[r] = max8(__float_as_uint(v[r]) & 0x7fffffffu);
+  float amax = __uint_as_float(m[0]);
+#pragma unroll
+  for (int r = 1; r < 4; r++)
+    if (__uint_as_float(m[r]) > amax) amax = __uint_as_float(m[r]);
+  Quantized4 o;
+  o.scale = fdiv(amax, bias == 0 ? 127.0f : 63.0f);
+  const float inv = o.scale > 0.0f ? fdiv(1.0f, o.scale) : 0.0f;
+  uint32_t q[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    int32_t tq;  // v_cvt_i32_f32 is i32.trunc_sat_f32_s (saturating, NaN 0)
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(tq) : "v"(rintf(fmul(v[r], inv))));
+    const int32_t sum = (int32_t)((uint32_t)tq + (uint32_t)bias);  // i32x4.add wraps
+    q[r] = (uint32_t)min(max(sum, -128), 127);                     // the two saturating narrowings
+  }
+  o.d = perm(perm(q[3], q[2], 0x0400u), perm(q[1], q[0], 0x0400u), 0x05040100u);
+  o.s4 = sdot4((int32_t)o.d, 0x01010101, 0);
+  o.s8 = o.s4 + dpp<0xB1>(o.s4);
+  o.s16 = o.s8 + dpp<0x4E>(o.s8);
+  return o;
+}
+
 // kernels/kernel/quantize.ts:124-151 for one group of 32 float32 values v: its 32 bytes (eight dwords, values
 // 4i..4i+3 in dword i) and its scale.  groupMax (quantize.ts:10-19): lane j's maximum of |values 4i + j| with a NaN
 // kept (a non-negative float's bits order as the float does, and every NaN's bits are above +inf's), then lanes 1..3
@@ -114,9 +159,6 @@ HQ_DEV void quantize_group(const float *p, int32_t bias, uint32_t q[8], float &s
   }
   quantize_values(v, bias, q, scale);
 }
-
-// v_perm_b32: byte i of the result is byte sel.i of {hi:lo} (0..3 from lo, 4..7 from hi)
-HQ_DEV uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) { return __builtin_amdgcn_perm(hi, lo, sel); }
 
 // the ternary codes of plane p of four bytes: (v >> 2p) & 3 a byte (kernels/ternary.ts:23-27).  The reference
 // shifts 16-bit lanes; with the mask 3 a 32-bit shift leaves the same bits (what a byte takes from its neighbour

@@ -51,8 +51,8 @@ struct JobPieces {
 };
 
 // where a kernel's activations come from: the caller's xq / xs in global memory (read through the L1), or a copy
-// of them the block makes in LDS
-enum Src { GLOBAL = 0, STAGED = 1 };
+// of them the block makes in LDS, or the block's own quantization of the float32 input into LDS (one token)
+enum Src { GLOBAL = 0, STAGED = 1, READY = 2 };
 
 // the LDS a block needs for T tokens of n activations (bytes, then float32 scales)
 HQ_HOST_DEV constexpr int64_t act_lds_bytes(int T, int n) { return (int64_t)T * (n + 4 * (n / 32)); }
@@ -69,6 +69,26 @@ HQ_DEV void fill_acts(const Job &J, char *lq, float *ls) {
     dst[0] = *(const uint4 *)src;
     dst[1] = *(const uint4 *)(src + 16);
     ls[t * ng + g] = ((const float *)(J.xs + t * J.sframe))[g];
+  }
+  __syncthreads();
+}
+
+// READY: fill the block's LDS with quantize_x (bias 64) of the n values at x, as fill_acts lays them out; with `keep` the
+// caller's xq and xs are written too
+HQ_DEV void fill_ready(const char *x, const Job &J, char *lq, float *ls, bool keep) {
+  const int n = J.n;
+  for (int first = 0; first < n; first += 4 * (int)blockDim.x) {
+    const int at = first + 4 * (int)threadIdx.x;
+    const bool live = at < n;  // (whole groups of 8 lanes: n is a multiple of 32)
+    const Quantized4 o = quantize4(*(const float4 *)(x + 4 * (int64_t)(live ? at : 0)), 64);
+    if (live) {
+      *(uint32_t *)(lq + at) = o.d;
+      if (keep) *(uint32_t *)((char *)J.xq + at) = o.d;
+      if ((threadIdx.x & 7) == 0) {
+        ls[at >> 5] = o.scale;
+        if (keep) ((float *)J.xs)[at >> 5] = o.scale;
+      }
+    }
   }
   __syncthreads();
 }
@@ -364,7 +384,7 @@ struct RelaxedChunk {
 // the relaxed_threads / RL rows of tile `blk` of job `jb` (its row range cut into tiles in order).  STAGED: first
 // make the block's LDS copy of the activations, while the first weights are in flight
 template <int PACK, int T, bool WC, int SRC, int RL, int U1, int NT, bool CACHED>
-HQ_DEV void relaxed_tile(const Job &J, int blk, char *lds) {
+HQ_DEV void relaxed_tile(const Job &J, int blk, char *lds, const char *x = nullptr, bool keep = false) {
   const int lane = threadIdx.x & (RL - 1);
   constexpr int rows = NT / RL;
   const int row_u = J.r0 + blk * rows + (int)(threadIdx.x / RL);
@@ -399,9 +419,10 @@ HQ_DEV void relaxed_tile(const Job &J, int blk, char *lds) {
   constexpr int U = Chunk::U;
   const int steps = (ng4 + RL - 1) / RL;
   Chunk a, b;
-  if (SRC == STAGED) {
+  if (SRC != GLOBAL) {
     if (steps > 0) a.load_w(wrow, srow, crow, 0, lane, ng4);  // the first weights in flight during the staging
-    fill_acts<T>(J, lds, (float *)(lds + T * J.n));
+    if (SRC == STAGED) fill_acts<T>(J, lds, (float *)(lds + T * J.n));
+    else fill_ready(x, J, lds, (float *)(lds + J.n), keep);
     if (steps > 0) a.load_x(A, 0, lane, ng4);
   } else if (Chunk::PAIRED) {
     if (steps > 0) a.load_paired(wb, sb, cb, rb, gb, A, 0, lane, ng4);
@@ -509,6 +530,18 @@ __global__ __launch_bounds__(NT) void gemv_relaxed(
   int jb, blk;
   block_job<BY>(batch, jb, blk);
   relaxed_tile<PACK, T, WC, SRC, RL, U1, NT, CACHED>(batch.job[jb], blk, lds);
+}
+
+// One token of int8 / int6 from its float32 input in one launch (kReadyThreads a block, 16-lane rows): every block
+// quantizes the input into its LDS while its first weights are in flight, the first block also into the caller's xq and
+// xs.  For launches so small that a quantize_x launch of their own costs more (gemv_ready_takes).
+constexpr int kReadyThreads = 128;
+template <int PACK, bool WC>
+__global__ __launch_bounds__(kReadyThreads) void gemv_ready(const char *x, GemvBatch batch) {
+  extern __shared__ __align__(16) char lds[];
+  const int jb = job_of(batch, (int)blockIdx.x);
+  relaxed_tile<PACK, 1, WC, READY, 16, 4, kReadyThreads, true>(batch.job[jb], (int)blockIdx.x - batch.block0[jb], lds, x,
+                                                               blockIdx.x == 0);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1208,6 +1241,44 @@ hipError_t launch_batch(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s
   }
 }
 }  // namespace
+
+// gemv_ready's launches: inputs of at most kReadyWidth values, weights of at most kReadyWeights bytes as int8.  Measured (a
+// layer of int8 decode replayed as a graph, us, quantize_x apart / in the launch): 288 wide 15.4 / 11.1, 512 wide (1408 down)
+// 17.0 / 13.5, 1024 wide 20.3 / 18.7 (its 4608-wide down projection in the launch: 22.0), 2048 wide 27.6 / 29.1: a block's
+// quantization grows with the width, and with it the blocks that repeat it.
+constexpr int32_t kReadyWidth = 1536;
+constexpr int64_t kReadyWeights = 10 << 20;
+bool gemv_ready_takes(Kind kind, const Job *jobs, int32_t njobs) {
+  if ((kind != Q8R && kind != Q6R) || njobs < 1 || njobs > kMaxJobs) return false;
+  int64_t bytes = 0;
+  for (int j = 0; j < njobs; j++) {
+    if (jobs[j].count != 1 || jobs[j].n != jobs[0].n || (jobs[j].wc != nullptr) != (jobs[0].wc != nullptr)) return false;
+    bytes += (int64_t)(jobs[j].r1 - jobs[j].r0) * jobs[j].n;
+  }
+  return jobs[0].n <= kReadyWidth && bytes <= kReadyWeights;
+}
+
+hipError_t launch_gemv_ready(Kind kind, const char *x, const Job *jobs, int32_t njobs, hipStream_t s) {
+  GemvBatch b{};
+  constexpr int rows = kReadyThreads / 16;
+  int blocks = 0;
+  for (int j = 0; j < njobs; j++) {
+    b.job[j] = jobs[j];
+    b.block0[j] = blocks;
+    blocks += (jobs[j].r1 - jobs[j].r0 + rows - 1) / rows;
+  }
+  b.block0[njobs] = blocks;
+  for (int j = njobs + 1; j <= kMaxJobs; j++) b.block0[j] = INT32_MAX;
+  b.njobs = njobs;
+  const size_t lds = (size_t)act_lds_bytes(1, jobs[0].n);
+  const dim3 grid(blocks), block(kReadyThreads);
+  const bool wc = jobs[0].wc != nullptr;
+  if (kind == Q8R && wc) hipLaunchKernelGGL((gemv_ready<8, true>), grid, block, lds, s, x, b);
+  else if (kind == Q8R) hipLaunchKernelGGL((gemv_ready<8, false>), grid, block, lds, s, x, b);
+  else if (wc) hipLaunchKernelGGL((gemv_ready<6, true>), grid, block, lds, s, x, b);
+  else hipLaunchKernelGGL((gemv_ready<6, false>), grid, block, lds, s, x, b);
+  return hipGetLastError();
+}
 
 // jobs: one kind, one token count (1..4), one wc-ness (all with corrections or all without)
 hipError_t launch_gemv(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s) {

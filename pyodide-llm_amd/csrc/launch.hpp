@@ -69,6 +69,10 @@ inline int cu_count() {
 // GEMV-shaped products (every job of one kind and one token count, 1..4; up to kMaxJobs jobs a launch)
 constexpr int kMaxJobs = 8;
 hipError_t launch_gemv(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s);
+// one token's int8 / int6 jobs from their float32 input x (16-byte aligned; xq and xs written too), of one xq / xs and
+// one wc-ness: whether such a launch is worth it, and the launch
+bool gemv_ready_takes(Kind kind, const Job *jobs, int32_t njobs);
+hipError_t launch_gemv_ready(Kind kind, const char *x, const Job *jobs, int32_t njobs, hipStream_t s);
 
 // llama.cpp's blocks: the tables from the codebooks row; a token's sums of 16 and 8 after its scales (count tokens,
 // frame apart); a row as float32; the products (jobs of the sb kinds, 1..4 tokens, up to kMaxJobs a launch); the
@@ -77,6 +81,10 @@ hipError_t launch_sb_tables(uint8_t *area, const uint8_t *codebooks, hipStream_t
 hipError_t launch_sums_x(char *xs, const char *xq, int32_t n, int32_t count, int64_t frame, hipStream_t s);
 hipError_t launch_sb_row(float *out, const char *w, const uint8_t *tab, int32_t n, int32_t type, hipStream_t s);
 hipError_t launch_sb(const Job *jobs, int32_t njobs, hipStream_t s);
+// one token's jobs from their float32 input x (16-byte aligned; xq and xs written too; NULL: launch_sb), of one xq / xs:
+// whether launch_sb_ready takes them
+bool sb_ready_takes(const Job *jobs, int32_t njobs);
+hipError_t launch_sb_ready(const char *x, const Job *jobs, int32_t njobs, hipStream_t s);
 // a prompt of kSbTileMin tokens or more of one job (the sb kinds), on the matrix cores: every (row, token)
 // launch_sb's number
 constexpr int kSbTileMin = 16;

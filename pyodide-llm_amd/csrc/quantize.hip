@@ -48,28 +48,11 @@ __global__ __launch_bounds__(256) void quantize_kernel(char *xq, char *xs, const
 // The activations' whole preparation in one launch (ready(), src/runtime/jobs.ts:376-395, 421-424): quantize_x's bytes
 // and scales, and per MODE interleave()'s planes and negated group sums (kMode 1: ternary, binary) or sums_x's int16
 // sums of 16 and 8 (kMode 2: llama.cpp's blocks).  A lane takes 4 consecutive values (one 16-byte load, one 4-byte
-// store), 8 lanes a group of 32: value 4 i + r is component r of the group's lane i, so a component's largest |value|
-// over the 8 lanes is groupMax's lane r (a non-negative float's bits order as the float does, and every NaN's are above
-// +inf's).
+// store), 8 lanes a group of 32 (quantize4).
 // Bound by HBM for a prompt and by the launch for a token.  Against quantize_kernel (a value a lane, a byte a store) and
 // interleave's or sums_x's own launch, through hq_matmuls: a token of the 27B ternary gate/up and down 24.1 -> 20.7 us,
 // of the 8B Q4_K ones 34.5 -> 30.9, an 8B layer's 2048 tokens 1902 -> 1811 us, a 1B layer's 512 239 -> 223.
 constexpr int kReadyValues = 1024;  // a block's values: 256 threads of 4
-
-// the largest bits of the 8 lanes of a group
-HQ_DEV uint32_t max8(uint32_t m) {
-  m = max(m, (uint32_t)dpp<0xB1>((int32_t)m));   // quad_perm [1, 0, 3, 2]
-  m = max(m, (uint32_t)dpp<0x4E>((int32_t)m));   // quad_perm [2, 3, 0, 1]
-  return max(m, (uint32_t)dpp<0x141>((int32_t)m));  // row_half_mirror
-}
-
-// the bytes of quantize_values (common.hpp) for one value: v_cvt_i32_f32 is i32.trunc_sat_f32_s (saturating, NaN 0)
-HQ_DEV int32_t quantized(float v, float inv, int32_t bias) {
-  int32_t tq;
-  asm("v_cvt_i32_f32 %0, %1" : "=v"(tq) : "v"(rintf(fmul(v, inv))));
-  const int32_t q = (int32_t)((uint32_t)tq + (uint32_t)bias);  // i32x4.add wraps
-  return min(max(q, -128), 127);                               // the two saturating narrowings
-}
 
 template <int MODE>
 __global__ __launch_bounds__(256) void ready_kernel(char *xq, char *xs, const char *x, int32_t n, int32_t bias,
@@ -80,44 +63,29 @@ __global__ __launch_bounds__(256) void ready_kernel(char *xq, char *xs, const ch
   const int64_t t = blockIdx.y;
   const int g = at >> 5, lane = threadIdx.x & 63;
   const float4 f = *(const float4 *)(x + t * x_stride + 4 * (int64_t)(live ? at : 0));
-  const float v[4] = {f.x, f.y, f.z, f.w};
-  uint32_t m[4];
-#pragma unroll
-  for (int r = 0; r < 4; r++) m[r] = max8(__float_as_uint(v[r]) & 0x7fffffffu);
-  float amax = __uint_as_float(m[0]);
-#pragma unroll
-  for (int r = 1; r < 4; r++)
-    if (__uint_as_float(m[r]) > amax) amax = __uint_as_float(m[r]);
-  const float scale = fdiv(amax, bias == 0 ? 127.0f : 63.0f);
-  const float inv = scale > 0.0f ? fdiv(1.0f, scale) : 0.0f;
-  uint32_t q[4];
-#pragma unroll
-  for (int r = 0; r < 4; r++) q[r] = (uint32_t)quantized(v[r], inv, bias);
-  const uint32_t d = perm(perm(q[3], q[2], 0x0400u), perm(q[1], q[0], 0x0400u), 0x05040100u);
+  const Quantized4 o = quantize4(f, bias);
   char *to = xq + t * frame, *st = xs + t * frame;
-  if (live && (lane & 7) == 0) ((float *)st)[g] = scale;
+  if (live && (lane & 7) == 0) ((float *)st)[g] = o.scale;
   if (MODE == 0) {
-    if (live) *(uint32_t *)(to + at) = d;
+    if (live) *(uint32_t *)(to + at) = o.d;
     return;
   }
-  int32_t s = sdot4((int32_t)d, 0x01010101, 0);  // the sum of 4, then of 8, 16 and 32
-  const int32_t s8 = s + dpp<0xB1>(s), s16 = s8 + dpp<0x4E>(s8);
   if (MODE == 1) {
-    const int32_t s32 = s16 + dpp<0x141>(s16);
+    const int32_t s32 = o.s16 + dpp<0x141>(o.s16);
     if (live && (lane & 7) == 0) ((int32_t *)st)[(n >> 5) + g] = -s32;
     // byte 16 p + c of a block of 64 is value 4 c + p: the quad m of the block's 16 lanes holds c = 4 m .. + 3, and
     // its lane p gathers byte p of the four lanes into the dword at 16 p + 4 m
-    const uint32_t q0 = (uint32_t)dpp<0x00>((int32_t)d), q1 = (uint32_t)dpp<0x55>((int32_t)d);
-    const uint32_t q2 = (uint32_t)dpp<0xAA>((int32_t)d), q3 = (uint32_t)dpp<0xFF>((int32_t)d);
+    const uint32_t q0 = (uint32_t)dpp<0x00>((int32_t)o.d), q1 = (uint32_t)dpp<0x55>((int32_t)o.d);
+    const uint32_t q2 = (uint32_t)dpp<0xAA>((int32_t)o.d), q3 = (uint32_t)dpp<0xFF>((int32_t)o.d);
     const uint32_t p = lane & 3, sel = p | ((4 + p) << 8);
-    const uint32_t o = perm(perm(q3, q2, sel), perm(q1, q0, sel), 0x05040100u);
-    if (live) *(uint32_t *)(to + (at & ~63) + 16 * p + (lane & 12)) = o;
+    const uint32_t plane = perm(perm(q3, q2, sel), perm(q1, q0, sel), 0x05040100u);
+    if (live) *(uint32_t *)(to + (at & ~63) + 16 * p + (lane & 12)) = plane;
   } else {
     int16_t *a16 = (int16_t *)(st + 4 * (n >> 5)), *a8 = a16 + (n >> 4);
     if (live) {
-      *(uint32_t *)(to + at) = d;
-      if ((lane & 1) == 0) a8[at >> 3] = (int16_t)s8;
-      if ((lane & 3) == 0) a16[at >> 4] = (int16_t)s16;
+      *(uint32_t *)(to + at) = o.d;
+      if ((lane & 1) == 0) a8[at >> 3] = (int16_t)o.s8;
+      if ((lane & 3) == 0) a16[at >> 4] = (int16_t)o.s16;
     }
   }
 }

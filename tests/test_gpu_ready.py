@@ -6,6 +6,7 @@ import pytest
 
 from gpu_util import Arena, same_bits
 from models import F
+from streams import pack6
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +87,50 @@ def test_quantize_x_anywhere(pkg, arena, oracle, x_off, xq_off):
     assert np.array_equal(got[xq_off:xq_off + n], want_q)
     assert np.all(got[:xq_off] == 0xAA) and np.all(got[xq_off + n:] == 0xAA)
     assert same_bits(arena.get(xs, F, n // 32), want_s)
+
+
+@pytest.mark.parametrize("kind,n", [("matmul_q8r", 512), ("matmul_q6r", 1536), ("matmul_sbr", 1280)])
+@pytest.mark.parametrize("place", ["apart", "over x"])
+def test_one_token_from_its_float32_input(pkg, arena, oracle, kind, n, place):
+    """one token's products with the input readied in their own launch; outputs over the input take the input apart first
+    (the launch's blocks would read what others of it write)"""
+    from pyodide_llm_amd import jobs
+    rng = np.random.default_rng(n)
+    ng = n // 32
+    x = rng.standard_normal(n).astype(F)
+    rows = (70, 33)
+    acts = arena.alloc(8 * n, fill=np.zeros(8 * n, np.uint8))
+    ax, b = arena.put(x), acts + n
+    outs = [ax if place == "over x" else arena.alloc(4 * r, fill=np.full(r, -7, F)) for r in rows]
+    if place == "over x":
+        outs[1] = ax + 4 * rows[0]
+    q, scales = oracle.quantize_x(x, 0 if kind == "matmul_sbr" else 64)
+    table, wants = [], []
+    if kind == "matmul_sbr":
+        import blocks_model as bm
+        row = bm.codebooks(rng)
+        tab, area = oracle.sb_tables(row), arena.alloc(34992)
+        assert pkg.library().hq_sb_tables_ex(area, arena.put(row), None) == 0
+        acts_area = oracle.sums_x(q.view(np.int8), scales)
+    for r, out in zip(rows, outs):
+        if kind == "matmul_sbr":
+            w = bm.random_blocks(rng, 12, r * (n // 256))
+            args = (arena.put(w), area, 12)
+            wants.append(oracle.matmul_sbr(q.view(np.int8), acts_area, w, tab, n, 12))
+        else:
+            ws = (np.abs(rng.standard_normal(r * ng)) * 0.02).astype(F)
+            if kind == "matmul_q6r":
+                w = pack6((4 * rng.integers(-32, 32, r * n)).astype(np.int8))
+                wc, product = oracle.six_sums(w), oracle.matmul_q6r
+            else:
+                w = rng.integers(-128, 128, r * n).astype(np.int8)
+                wc, product = oracle.int8_sums(w), oracle.matmul_q8r
+            args = (arena.put(w), arena.put(ws), arena.put(wc))
+            wants.append(product(q, scales, w, ws, wc, n))
+        table.append(jobs.job(kind, out, acts, b, *args, n, rows=r))
+    L = pkg.library()
+    assert jobs.matmuls(L, ax, 4 * n, table) == 0, L.hq_last_error_message()
+    for out, r, want in zip(outs, rows, wants):
+        assert same_bits(arena.get(out, F, r), want)
+    assert np.array_equal(arena.get(acts, np.uint8, n), q.view(np.uint8))
+    assert same_bits(arena.get(b, F, ng), scales)

@@ -35,14 +35,17 @@ bool tile_offsets_fit(hq::Kind kind, const hq::Job &j) {
   return 64 * j.frame + j.n < kLimit && 64 * j.sframe + scales < kLimit && 128 * row_bytes < kLimit;
 }
 
+bool blocks_tile_fits(const hq::Job &j) {
+  return j.frame > 0 && j.sframe > 0 && j.frame < hq::kSbTileFrameMax && j.sframe < hq::kSbTileFrameMax;
+}
+
 // Which kernels take a job: 1 the matrix-core tile, 0 the token kernel (4 tokens a launch).  The tiles keep a lane's
 // offsets within a tile in 32 bits: 64 tokens of activations (frame and sframe bytes apart: 128 for the blocks' tile)
 // and 128 rows of weights, so a job whose tile would reach 4 GiB from its first byte takes the token kernel, whose
 // addresses are 64-bit.
 int32_t path_of(hq::Kind kind, const hq::Job &j) {
   if (hq::blocks_kind(kind)) {
-    return j.count >= hq::kSbTileMin && j.frame > 0 && j.sframe > 0 && j.frame < hq::kSbTileFrameMax &&
-           j.sframe < hq::kSbTileFrameMax;
+    return j.count >= hq::kSbTileMin && blocks_tile_fits(j);
   }
   return j.count >= kGemmMinTokens && hq::gemm_supported(kind) && tile_offsets_fit(kind, j);
 }
@@ -226,6 +229,15 @@ int32_t run_together(std::vector<hq::Job> &jobs, hq::Kind kind, Launch launch) {
   return HQ_OK;
 }
 
+// The blocks' jobs that take the matrix-core tile: what would be three launches or more of the token kernel (4 tokens
+// each), or two of them for a large matrix.  Measured (the 8B gate/up and down, us, token kernel / tile): IQ3_S at 5 tokens
+// 131 / 144, 6 tokens 158 / 144, 9 tokens 209 / 144, 15 tokens 336 / 144; a 1024-wide model's IQ2_XXS at 8 tokens 34 / 36, 9
+// tokens 48 / 37, 15 tokens 57 / 37.
+bool blocks_tile_takes(const hq::Job &j) {
+  const bool large = (int64_t)(j.r1 - j.r0) * j.n >= (int64_t)1 << 23;
+  return j.count >= (large ? 6 : 9) && blocks_tile_fits(j);
+}
+
 // runs jobs of one kind: few-token jobs and GEMV jobs (up to 4 tokens; more in slices of 4) batched in launches of up to kMaxJobs,
 // GEMM jobs one a launch
 int32_t run_blocks(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s) {
@@ -239,7 +251,7 @@ int32_t run_blocks(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t 
       continue;
     }
     // a prompt: the matrix-core tile (its offsets within a tile of tokens are 32-bit: frames under 16 MB)
-    if (path_of(kind, j)) {
+    if (blocks_tile_takes(j)) {
       const int32_t st = hip_status(hq::launch_sb_tile(j, s), kind_name(kind));
       if (st) return st;
       continue;

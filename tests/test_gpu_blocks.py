@@ -372,3 +372,31 @@ def test_q4k_tiles(pkg, arena, oracle, setup, n, rows, tokens):
         got = arena.get(out, F, tokens * rows).reshape(tokens, rows)
         want = oracle.matmul_sbr(*ready[-1], mats[0], tab, n, 12)
         assert np.all(got[:, :5] == -7) and np.all(got[:, rows - 3:] == -7) and same_bits(got[-1, 5:rows - 3], want[5:rows - 3])
+
+
+@pytest.mark.parametrize("name,t", [("IQ2_XS", 17), ("IQ1_M", 29), ("Q2_K", 10), ("IQ4_XS", 23)])
+@pytest.mark.parametrize("rows,tokens", [(40, 8), (40, 9), (16400, 6)])
+def test_few_tokens_on_the_tile(pkg, arena, oracle, setup, name, t, rows, tokens):
+    """both sides of the line between the token kernel and the tile below 16 tokens (n 512: 16400 rows are a large
+    matrix), every (row, token) the oracle's"""
+    row, tab = setup
+    n = 512
+    area = arena.alloc(34992)
+    L = pkg.library()
+    assert L.hq_sb_tables_ex(area, arena.put(row), None) == 0
+    rng = np.random.default_rng(t + tokens)
+    frame = 2 * n
+    buf = np.zeros((tokens, frame), np.uint8)
+    ready = []
+    for i in range(tokens):
+        q, area_t = token_area(oracle, rng, n, 1.0 + i)
+        buf[i, :n], buf[i, n:n + area_t.size] = q.view(np.uint8), area_t.view(np.uint8)
+        ready.append((q, area_t))
+    blocks = bm.random_blocks(rng, t, rows * (n // 256))
+    a = arena.put(buf)
+    out = arena.alloc(4 * rows * tokens, fill=np.full(rows * tokens, -7, F))
+    assert L.hq_matmul_sbr_tile_ex(out, a, a + n, arena.put(blocks), area, n, 0, rows, tokens, 4 * rows, frame, t, None) == 0
+    got = arena.get(out, F, rows * tokens).reshape(tokens, rows)
+    for i in (0, tokens - 1):
+        want = oracle.matmul_sbr(*ready[i], blocks, tab, n, t)
+        assert same_bits(got[i], want), (i, first_difference(got[i], want))

@@ -238,8 +238,8 @@ bool blocks_tile_takes(const hq::Job &j) {
   return j.count >= (large ? 6 : 9) && blocks_tile_fits(j);
 }
 
-// runs jobs of one kind: few-token jobs and GEMV jobs (up to 4 tokens; more in slices of 4) batched in launches of up to kMaxJobs,
-// GEMM jobs one a launch
+// runs jobs of one kind: few-token jobs and GEMV jobs (up to 4 tokens; more in slices of 4) and prompt tiles,
+// batched in launches of up to kMaxJobs
 int32_t run_blocks(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s) {
   // up to 4 tokens a launch (a prompt in slices of 4: every (row, token) the token kernel's number), jobs of one
   // block type, one token count and one tables' area together
@@ -285,7 +285,7 @@ int32_t run_blocks(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t 
 int32_t run_jobs(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s) {
   if (hq::blocks_kind(kind)) return run_blocks(kind, jobs, s);
   std::vector<hq::Job> gemv[hq::kGemvMaxTokens + 1][2];  // by token count, by wc-ness
-  std::vector<hq::Job> few;
+  std::vector<hq::Job> few, tiles;
   for (const hq::Job &j : jobs) {
     if (j.r1 == j.r0 || j.count == 0) continue;
     if (few_tokens(kind, j)) {
@@ -293,8 +293,7 @@ int32_t run_jobs(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s)
       continue;
     }
     if (path_of(kind, j)) {
-      const int32_t st = hip_status(hq::launch_gemm(kind, j, s), kind_name(kind));
-      if (st) return st;
+      tiles.push_back(j);
       continue;
     }
     for (int32_t t0 = 0; t0 < j.count; t0 += hq::kGemvMaxTokens) {
@@ -306,6 +305,8 @@ int32_t run_jobs(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s)
       gemv[part.count][part.wc != nullptr].push_back(part);
     }
   }
+  if (int32_t st = run_together(tiles, kind, [&](const hq::Job *same, int32_t m) { return hq::launch_gemm(kind, same, m, s); }))
+    return st;
   if (int32_t st = run_together(few, kind, [&](const hq::Job *same, int32_t m) { return hq::launch_few(kind, same, m, s); }))
     return st;
   for (int c = 1; c <= hq::kGemvMaxTokens; c++)

@@ -71,6 +71,23 @@ constexpr int AHEAD = RING - 1;   // stages loaded beyond the one computed
 // blocks)
 template <int R> constexpr int ring_of() { return R == 32 ? 3 : 4; }
 
+// a launch's jobs (one kind and token count, all with wc or none), their tiles one job's after the other's
+struct GemmBatch {
+  Job job[kMaxJobs];
+  int32_t block0[kMaxJobs];  // the first tile of each job (INT32_MAX past the last)
+  int32_t blocks[kMaxJobs];
+};
+// the block's job and its tile of it (row tile rb of R rows, token tile tb)
+template <int R>
+HQ_DEV const Job &batch_tile(const GemmBatch &batch, int &rb, int &tb) {
+  int jb = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxJobs; i++) jb += (int)blockIdx.x >= batch.block0[i] ? 1 : 0;
+  const Job &J = batch.job[jb];
+  tile_of((int)blockIdx.x - batch.block0[jb], batch.blocks[jb], (J.r1 - J.r0 + R - 1) / R, rb, tb);
+  return J;
+}
+
 HQ_DEV v16i zero16i() {
   v16i z;
 #pragma unroll
@@ -592,13 +609,13 @@ HQ_DEV void q_chain(const Job &J, int row0, int tok0, int M, int stages, StageQ<
 }
 
 template <int PACK, bool WC, bool WIDE, int R>
-__global__ __launch_bounds__(QT, ring_of<R>() == 3 ? 3 : 2) void gemm_relaxed(Job J) {
+__global__ __launch_bounds__(QT, ring_of<R>() == 3 ? 3 : 2) void gemm_relaxed(GemmBatch batch) {
   __shared__ StageQ<R> b0, b1, b2;
   __shared__ StageQ<R> b3x[1];  // not allocated for a ring of 3 (never used then)
   StageQ<R> &b3 = ring_of<R>() == 3 ? b2 : b3x[0];
-  const int M = J.count;
   int rb, tb;
-  tile_of(blockIdx.x, gridDim.x, (J.r1 - J.r0 + R - 1) / R, rb, tb);
+  const Job &J = batch_tile<R>(batch, rb, tb);
+  const int M = J.count;
   const int row0 = J.r0 + rb * R, tok0 = tb * BT;
   const int lane = threadIdx.x & 63;
   const int chain = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -829,13 +846,13 @@ HQ_DEV void t_step(Ternary<BIN, R> &L, const StageT<R> &cur, StageT<R> &next, in
 
 // the tile's stages, the four parts' chains added in order ((p0 + p1) + p2) + p3 (math.ts:7-9), part 3's waves storing
 template <bool BIN, int R>
-__global__ __launch_bounds__(64 * 4 * (R / 32)) void gemm_ternary(Job J) {
+__global__ __launch_bounds__(64 * 4 * (R / 32)) void gemm_ternary(GemmBatch batch) {
   __shared__ StageT<R> b0, b1, b2, b3;
   __shared__ __attribute__((aligned(16))) char junk[1024];
+  int rb, tb;
+  const Job &J = batch_tile<R>(batch, rb, tb);
   const int M = J.count;
   const int groups = J.n >> 7;
-  int rb, tb;
-  tile_of(blockIdx.x, gridDim.x, (J.r1 - J.r0 + R - 1) / R, rb, tb);
   const int row0 = J.r0 + rb * R, tok0 = tb * BT;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -875,15 +892,37 @@ __global__ __launch_bounds__(64 * 4 * (R / 32)) void gemm_ternary(Job J) {
   }
 }
 
+// the tiles of `rows` rows that the jobs take
+int64_t tiles_of(const Job *jobs, int32_t njobs, int rows, int token_tiles) {
+  int64_t n = 0;
+  for (int j = 0; j < njobs; j++) n += (int64_t)((jobs[j].r1 - jobs[j].r0 + rows - 1) / rows) * token_tiles;
+  return n;
+}
+// Several jobs a launch (q, k and v; gate and up): a launch each left its last round of tiles part empty, and small
+// ones most of the GPU (through hq_matmuls, us: a 1B layer of 512 tokens 223 -> 200, the 27B ternary gate/up and down of
+// 251 tokens 408 -> 396, an 8B layer of 2048 tokens 1811 -> 1803).
+GemmBatch batch_of(const Job *jobs, int32_t njobs, int rows, int token_tiles, int64_t &blocks) {
+  GemmBatch b{};
+  blocks = 0;
+  for (int j = 0; j < kMaxJobs; j++) b.block0[j] = INT32_MAX;
+  for (int j = 0; j < njobs; j++) {
+    b.job[j] = jobs[j];
+    b.block0[j] = (int32_t)blocks;
+    b.blocks[j] = (int32_t)tiles_of(jobs + j, 1, rows, token_tiles);
+    blocks += b.blocks[j];
+  }
+  return b;
+}
+
 // The ternary tile's rows for a launch: 96 where that costs less, a launch costing its rounds of tiles over the CUs
 // (one block a CU) times the tile's rows times its cost a row (a 96-row tile of 12 waves does 1.155 times the 128-row
 // tile's time a row, measured over launches of many rounds: 348 against 402 TOPS).  27B at M = 256: gate/up 544
 // tiles of 128 rows (3 rounds, the last an eighth full) against 728 of 96 (3 rounds), 276 -> 331 TOPS; down 160 of
 // 128 (96 CUs idle) against 216 of 96, 276 -> 329; at M = 1024 both keep 128 rows.
-int ternary_rows(int rows, int token_tiles) {
+int ternary_rows(const Job *jobs, int32_t njobs, int token_tiles) {
   const int64_t cus = cu_count();
-  const int64_t r128 = ((int64_t)((rows + 127) / 128) * token_tiles + cus - 1) / cus;
-  const int64_t r96 = ((int64_t)((rows + 95) / 96) * token_tiles + cus - 1) / cus;
+  const int64_t r128 = (tiles_of(jobs, njobs, 128, token_tiles) + cus - 1) / cus;
+  const int64_t r96 = (tiles_of(jobs, njobs, 96, token_tiles) + cus - 1) / cus;
   return 96.0 * 1.155 * (double)r96 < 128.0 * (double)r128 ? 96 : 128;
 }
 
@@ -895,19 +934,28 @@ bool wide_scales(const Job &j) {
 }
 
 template <bool BIN, int R>
-void launch_ternary(const Job &job, int token_tiles, hipStream_t s) {
-  const dim3 grid(((job.r1 - job.r0 + R - 1) / R) * token_tiles);
-  hipLaunchKernelGGL((gemm_ternary<BIN, R>), grid, dim3(8 * R), 0, s, job);
+hipError_t launch_ternary(const Job *jobs, int32_t njobs, int token_tiles, hipStream_t s) {
+  int64_t blocks;
+  const GemmBatch b = batch_of(jobs, njobs, R, token_tiles, blocks);
+  if (blocks > INT32_MAX) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((gemm_ternary<BIN, R>), dim3((uint32_t)blocks), dim3(8 * R), 0, s, b);
+  return hipGetLastError();
 }
 
 template <int PACK, int R>
-void launch_relaxed(const Job &job, int token_tiles, hipStream_t s) {
-  const dim3 grid(((job.r1 - job.r0 + R - 1) / R) * token_tiles);
-  const bool wc = job.wc != nullptr, wide = wide_scales(job);
-  if (wc && wide) hipLaunchKernelGGL((gemm_relaxed<PACK, true, true, R>), grid, dim3(QT), 0, s, job);
-  else if (wc) hipLaunchKernelGGL((gemm_relaxed<PACK, true, false, R>), grid, dim3(QT), 0, s, job);
-  else if (wide) hipLaunchKernelGGL((gemm_relaxed<PACK, false, true, R>), grid, dim3(QT), 0, s, job);
-  else hipLaunchKernelGGL((gemm_relaxed<PACK, false, false, R>), grid, dim3(QT), 0, s, job);
+hipError_t launch_relaxed(const Job *jobs, int32_t njobs, int token_tiles, hipStream_t s) {
+  int64_t blocks;
+  const GemmBatch b = batch_of(jobs, njobs, R, token_tiles, blocks);
+  if (blocks > INT32_MAX) return hipErrorInvalidValue;
+  const dim3 grid((uint32_t)blocks);
+  const bool wc = jobs[0].wc != nullptr;
+  bool wide = true;
+  for (int j = 0; j < njobs; j++) wide = wide && wide_scales(jobs[j]);
+  if (wc && wide) hipLaunchKernelGGL((gemm_relaxed<PACK, true, true, R>), grid, dim3(QT), 0, s, b);
+  else if (wc) hipLaunchKernelGGL((gemm_relaxed<PACK, true, false, R>), grid, dim3(QT), 0, s, b);
+  else if (wide) hipLaunchKernelGGL((gemm_relaxed<PACK, false, true, R>), grid, dim3(QT), 0, s, b);
+  else hipLaunchKernelGGL((gemm_relaxed<PACK, false, false, R>), grid, dim3(QT), 0, s, b);
+  return hipGetLastError();
 }
 
 // 32-row tiles (three blocks a CU) where they cost less than 64-row tiles (two a CU): a launch costs its tiles over
@@ -917,9 +965,9 @@ void launch_relaxed(const Job &job, int token_tiles, hipStream_t s) {
 // ways (the 8B layer at M = 2048, Llama-3.2-1B at 512, the 27B projections at 256) it picks the faster height each
 // time: 64 for the 8B shapes, the 1B gate/up and the 27B gate/up, 32 for the other 1B shapes and the 27B down.
 constexpr double kTile32 = 0.89;
-bool short_tiles(int rows, int token_tiles) {
+bool short_tiles(const Job *jobs, int32_t njobs, int token_tiles) {
   const double cus = (double)cu_count();
-  const double t64 = (double)((rows + 63) / 64) * token_tiles, t32 = (double)((rows + 31) / 32) * token_tiles;
+  const double t64 = (double)tiles_of(jobs, njobs, 64, token_tiles), t32 = (double)tiles_of(jobs, njobs, 32, token_tiles);
   return kTile32 * fmax(1.0, t32 / (3 * cus)) < fmax(1.0, t64 / (2 * cus));
 }
 
@@ -927,32 +975,22 @@ bool short_tiles(int rows, int token_tiles) {
 
 bool gemm_supported(Kind kind) { return kind == Q8R || kind == Q6R || signs_kind(kind); }
 
-hipError_t launch_gemm(Kind kind, const Job &job, hipStream_t s) {
-  const int rows = job.r1 - job.r0;
-  if (rows <= 0 || job.count <= 0) return hipSuccess;
-  const int token_tiles = (job.count + BT - 1) / BT;
+hipError_t launch_gemm(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s) {
+  if (njobs < 1 || njobs > kMaxJobs) return hipErrorInvalidValue;
+  const int tt = (jobs[0].count + BT - 1) / BT;
   switch (kind) {
-  case Q8R:
-    if (short_tiles(rows, token_tiles)) launch_relaxed<8, 32>(job, token_tiles, s);
-    else launch_relaxed<8, 64>(job, token_tiles, s);
-    break;
-  case Q6R:
-    if (short_tiles(rows, token_tiles)) launch_relaxed<6, 32>(job, token_tiles, s);
-    else launch_relaxed<6, 64>(job, token_tiles, s);
-    break;
+  case Q8R: return short_tiles(jobs, njobs, tt) ? launch_relaxed<8, 32>(jobs, njobs, tt, s) : launch_relaxed<8, 64>(jobs, njobs, tt, s);
+  case Q6R: return short_tiles(jobs, njobs, tt) ? launch_relaxed<6, 32>(jobs, njobs, tt, s) : launch_relaxed<6, 64>(jobs, njobs, tt, s);
   case T2R:
   case T2:
-    if (ternary_rows(rows, token_tiles) == 96) launch_ternary<false, 96>(job, token_tiles, s);
-    else launch_ternary<false, 128>(job, token_tiles, s);
-    break;
+    return ternary_rows(jobs, njobs, tt) == 96 ? launch_ternary<false, 96>(jobs, njobs, tt, s)
+                                               : launch_ternary<false, 128>(jobs, njobs, tt, s);
   case B1R:
   case B1:
-    if (ternary_rows(rows, token_tiles) == 96) launch_ternary<true, 96>(job, token_tiles, s);
-    else launch_ternary<true, 128>(job, token_tiles, s);
-    break;
+    return ternary_rows(jobs, njobs, tt) == 96 ? launch_ternary<true, 96>(jobs, njobs, tt, s)
+                                               : launch_ternary<true, 128>(jobs, njobs, tt, s);
   default: return hipErrorNotSupported;
   }
-  return hipGetLastError();
 }
 
 }  // namespace hq

@@ -109,9 +109,10 @@ hipError_t launch_outlier_columns(float *columns, const uint8_t *values, const u
                                   const Channels &ch, int32_t vocab, int32_t dim, int32_t group, hipStream_t s);
 hipError_t launch_take_channels(float *picked, float *x, const Channels &ch, hipStream_t s);
 
-// MFMA GEMM-shaped products (one job a launch; count > 4 tokens): the tiles of matmul_q8r_tile, matmul_q6r and
-// matmul_t2r_tile over a prompt.  Returns hipErrorNotSupported for a kind that has none.
-hipError_t launch_gemm(Kind kind, const Job &job, hipStream_t s);
+// MFMA GEMM-shaped products (jobs of some rows, of one token count and all with wc or none, up to kMaxJobs a launch): the
+// tiles of matmul_q8r_tile, matmul_q6r and matmul_t2r_tile over a prompt.  Returns hipErrorNotSupported for a kind that
+// has none.
+hipError_t launch_gemm(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s);
 
 // a few tokens on the matrix cores (few.hip): jobs of one kind (as launch_gemm's), one token count and all with wc or
 // none, up to kMaxJobs a launch

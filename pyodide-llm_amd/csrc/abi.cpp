@@ -51,15 +51,17 @@ int32_t path_of(hq::Kind kind, const hq::Job &j) {
 }
 
 // The jobs that few.hip's 16-token tiles take: from the token counts where its one pass over the weights beats the token
-// kernel's pass a 4 tokens, to those where gemm.hip's larger tiles fill the GPU.  Measured both ways (us, token kernel or
-// prompt tile / few.hip): an 8B layer of int8 at 4 tokens 65 / 76, 5 tokens 109 / 76, 64 tokens 214 / 168, 80 tokens
-// 200 / 206; the 27B MLP of int6 at 4 tokens 70 / 90, 64 tokens 225 / 212, of ternary at 2 tokens 37 / 66, 3 tokens 72 /
-// 67, 160 tokens 342 / 318, 192 tokens 347 / 356.
-constexpr int32_t kFewMin = 5, kFewMax = 64, kFewSignsMin = 3, kFewSignsMax = 160;
-bool few_tokens(hq::Kind kind, const hq::Job &j) {
+// kernel's pass a 4 tokens, to those where gemm.hip's larger tiles fill the GPU: more for a small phase (`weights`: those of
+// the phase's jobs of one kind).  Measured both ways (us, token kernel or prompt tile / few.hip): an 8B layer of int8 at 4
+// tokens 65 / 76, 5 tokens 109 / 76, 48 tokens 141 / 138, 64 tokens 154 / 168, a 350M one (9.4 M weights of gate and up) at
+// 64 tokens 56 / 53, 96 tokens 59 / 54, 128 tokens 60 / 60; the 27B MLP of int6 at 4 tokens 70 / 90, 32 tokens 176 / 148, 48
+// tokens 179 / 187; ternary's at 2 tokens 37 / 66, 3 tokens 72 / 67, 160 tokens 333 / 318, 192 tokens 339 / 350, a 1B
+// ternary layer (33 M) at 256 tokens 176 / 140, a 350M one at 400 tokens 117 / 93.
+bool few_tokens(hq::Kind kind, const hq::Job &j, int64_t weights) {
   const bool signs = hq::signs_kind(kind);
-  return hq::gemm_supported(kind) && j.count >= (signs ? kFewSignsMin : kFewMin) &&
-         j.count <= (signs ? kFewSignsMax : kFewMax) && tile_offsets_fit(kind, j);
+  const int32_t least = signs ? 3 : 5;
+  const int32_t most = signs ? (weights < (40 << 20) ? 400 : 160) : weights < (10 << 20) ? 96 : kind == hq::Q6R ? 40 : 48;
+  return hq::gemm_supported(kind) && j.count >= least && j.count <= most && tile_offsets_fit(kind, j);
 }
 
 int32_t fail(int32_t code, const char *fmt, ...) {
@@ -286,9 +288,11 @@ int32_t run_jobs(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s)
   if (hq::blocks_kind(kind)) return run_blocks(kind, jobs, s);
   std::vector<hq::Job> gemv[hq::kGemvMaxTokens + 1][2];  // by token count, by wc-ness
   std::vector<hq::Job> few, tiles;
+  int64_t weights = 0;
+  for (const hq::Job &j : jobs) weights += (int64_t)(j.r1 - j.r0) * j.n;
   for (const hq::Job &j : jobs) {
     if (j.r1 == j.r0 || j.count == 0) continue;
-    if (few_tokens(kind, j)) {
+    if (few_tokens(kind, j, weights)) {
       few.push_back(j);
       continue;
     }

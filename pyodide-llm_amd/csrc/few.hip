@@ -19,8 +19,8 @@
 //
 // Measured (through hq_matmuls, us, before: 4 tokens a gemv launch below 16 tokens, gemm.hip's tiles from 16): an 8B
 // layer of int8 without / with wc, 11 tokens 137 / 148 -> 78 / 80, 16 tokens 174 / 201 -> 80 / 83, 32 tokens 183 / 217 ->
-// 110 / 115, 64 tokens 214 / 244 -> 168 / 167; the 27B MLP of int6, 16 tokens 199 -> 96; of ternary, 4 tokens 96 -> 66, 16
-// tokens 212 -> 69, 64 tokens 233 -> 152, 128 tokens 321 -> 230.
+// 110 / 115; the 27B MLP of int6, 16 tokens 199 -> 96; of ternary, 4 tokens 96 -> 66, 16 tokens 212 -> 69, 64 tokens 233 ->
+// 152, 128 tokens 321 -> 230.
 // What bounds it (an 8B gate/up of 16 tokens, 30 us; copies with a part left out): the loads alone 28 us (the weights and
 // scales at HBM's rate are 20), the arithmetic alone 19, neither 10: a block's life has ~2 us of addresses, first loads
 // and sums that other blocks hide in part.  More tokens: the arithmetic (16 VALU instructions, 16 to 32 matrix-core

@@ -46,10 +46,10 @@ def matrix(rng, oracle, kind, rows, n):
     return w, ws, wc, lambda q, s, c=None: product(q, s, w, ws, wc if c is None else c, n)
 
 
-CASES = [("matmul_q8r", n, t, 0) for n in (32, 96, 288, 512, 1056, 1664) for t in (5, 16, 17, 33, 48, 64)] + \
+CASES = [("matmul_q8r", n, t, 0) for n in (32, 96, 288, 512, 1056, 1664) for t in (5, 16, 17, 33, 48, 64, 96)] + \
         [("matmul_q6r", n, t, 0) for n in (32, 288, 512, 1664) for t in (5, 16, 33, 49, 64)] + \
         [(k, n, t, 4) for k in ("matmul_q8r", "matmul_q6r") for n in (32, 512, 1664) for t in (5, 33)] + \
-        [(k, n, t, 0) for k in ("matmul_t2r", "matmul_b1r") for n in (128, 384, 512, 1664) for t in (3, 16, 17, 33, 160)]
+        [(k, n, t, 0) for k in ("matmul_t2r", "matmul_b1r") for n in (128, 384, 512, 1664) for t in (3, 16, 17, 33, 160, 400)]
 
 
 @pytest.mark.parametrize("kind,n,tokens,shift", CASES)

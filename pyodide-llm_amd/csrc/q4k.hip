@@ -13,8 +13,9 @@
 // block's bytes (in registers while this one is multiplied) go into the other of two buffers.
 //
 // Measured (the 8B gate/up and down through hq_matmuls, us, before: 4 tokens a launch of the token kernel below 16
-// tokens, blocks.hip's tile from 16): 4 tokens 108 -> 66, 15 tokens 353 -> 67, 16 tokens 187 -> 67, 32 tokens 190 -> 90, 64
-// tokens 254 -> 134, 333 tokens 911 -> 517, 512 tokens 1127 -> 721 (160 -> 250 TOPS).
+// tokens, blocks.hip's tile from 16): 4 tokens 108 -> 63, 15 tokens 353 -> 64, 16 tokens 187 -> 64, 32 tokens 190 -> 85,
+// 64 tokens 254 -> 115, 333 tokens 911 -> 477, 512 tokens 1127 -> 672 (160 -> 268 TOPS).  Of that, S times the integer
+// as a float32 product instead of v_mul_i32_i24, which issues slower: 333 tokens 521 -> 477, 512 tokens 728 -> 672.
 // What bounds a prompt: those 16 operations, 563 of a SIMD's cycles a pair and 32 x 32 outputs, beside 64 of the matrix
 // cores' (which add on this part: 459 TOPS at 2.2 GHz), and per step of a wave ~60 operations of scales and operands.
 // A few tokens: the steps' latency, one after the other down a row (56 steps of the down projection, 0.6 us each).
@@ -82,12 +83,13 @@ struct Q4kLoads {
     }
     if (tid < 4 * NT) {
       const int tok = tid >> 2, part = tid & 3;
-      float *to = (float *)(lds + (part & 2 ? L::V : L::XS)) + 4 * (part & 1) * NT + tok;
+      uint32_t *to = (uint32_t *)(lds + (part & 2 ? L::V : L::XS)) + 4 * (part & 1) * NT + tok;
+      const uint32_t sums = 0u - (uint32_t)(part >> 1);  // (a mask, not a branch an element)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         // two int16 sums of 16: the group's sum of 32
         const int32_t sum = (int32_t)(int16_t)(aux[i] & 0xffff) + (aux[i] >> 16);
-        to[i * NT] = part & 2 ? (float)sum : __int_as_float(aux[i]);
+        to[i * NT] = (__float_as_uint((float)sum) & sums) | ((uint32_t)aux[i] & ~sums);
       }
     }
 #pragma unroll
@@ -154,8 +156,7 @@ __global__ __launch_bounds__(256, 2) void gemm_q4k(Q4kBatch batch) {
     if (more) loads.load(J, rx, ra, rw, b + 1);
     // the rows' operands of groups k and k + 4: the nibbles, S, M, and the blocks' F and Fm
     Op B[RS][2];
-    int32_t S[RS][2];
-    float M[RS][2], F[RS], Fm[RS];
+    float S[RS][2], M[RS][2], F[RS], Fm[RS];
 #pragma unroll
     for (int sp = 0; sp < RS; sp++) {
       const char *row = st + L::RAW + (T * sp + at) * kQ4kBytes;
@@ -171,8 +172,8 @@ __global__ __launch_bounds__(256, 2) void gemm_q4k(Q4kBatch batch) {
       // bytes 4 + k, 8 + k, 12 + k: group k's S and M in the low six bits of the first two, group k + 4's low four bits
       // in the third's halves and their top two above those (types.ts:230-232)
       const uint32_t s = head.y >> (8 * k), m = head.z >> (8 * k), hi = head.w >> (8 * k);
-      S[sp][0] = (int32_t)(s & 63);
-      S[sp][1] = (int32_t)((hi & 15) | ((s >> 2) & 48));
+      S[sp][0] = (float)(s & 63);
+      S[sp][1] = (float)((hi & 15) | ((s >> 2) & 48));
       M[sp][0] = (float)(m & 63);
       M[sp][1] = (float)(((hi >> 4) & 15) | ((m >> 2) & 48));
       F[sp] = half_to_float(head.x & 0xffff);
@@ -200,7 +201,8 @@ __global__ __launch_bounds__(256, 2) void gemm_q4k(Q4kBatch batch) {
 #pragma unroll
           for (int i = 0; i < 4; i++) {
             const int r = 4 * m + i;
-            const float g = fadd(fmul((float)__mul24(S[sp][0], C[sp][0][r]), xa[i]), fmul((float)__mul24(S[sp][1], C[sp][1][r]), xb[i]));
+            // (S times the integer is exact in float32: below 2^22)
+            const float g = fadd(fmul(fmul(S[sp][0], (float)C[sp][0][r]), xa[i]), fmul(fmul(S[sp][1], (float)C[sp][1][r]), xb[i]));
             const float least = fadd(fmul(fmul(M[sp][0], va[i]), xa[i]), fmul(fmul(M[sp][1], vb[i]), xb[i]));
             acc[sp][h][r] = fadd(acc[sp][h][r], fsub(fmul(g, F[sp]), fmul(least, Fm[sp])));
             // (kept here: the compiler would sink the folds of every token half past the next block's stores, and spill)

@@ -19,6 +19,8 @@
 // A few tokens go 4 at a time through the same kernel (blocks_tile_takes in abi.cpp draws the line); a prompt through
 // the matrix-core tile below (gemm_sb): every (row, token) the token kernel's number either way.  (Q4_K whose blocks start
 // on 16 bytes takes q4k.hip's tiles from three tokens: the same numbers.)
+#include <type_traits>
+
 #include "common.hpp"
 #include "launch.hpp"
 #include "fold.hpp"
@@ -621,7 +623,7 @@ hipError_t launch_type(const SbBatch &b, int T, int L, size_t lds, hipStream_t s
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// the prompt tile (matmul_sbr_tile / matmul_sbw_tile for kSbTileMin tokens or more): a block takes 32 rows x NT
+// the prompt tile (matmul_sbr_tile / matmul_sbw_tile for the token counts of blocks_tile_takes): a block takes 32 rows x NT
 // tokens (NT 32, 64 or 128).  For each block of 256 weights it stages the tokens' activations (with their scales and
 // sums) and the rows' raw blocks into LDS, decodes the 32 blocks once (two chunks of 16 a thread, the token kernel's
 // decoder reading the LDS copy) into int8 tiles, and multiplies them on the matrix cores:
@@ -649,6 +651,13 @@ constexpr int SBT_PITCH = 256 + 16;  // an LDS row of a block's 256 bytes (16 mo
 
 template <int TY> constexpr bool tile_signed() { return has_signs<TY>(); }
 template <int TY> constexpr bool tile_split() { return TY == IQ2_XS || TY == IQ2_S || TY == IQ1_M; }
+// whether S times a group's integer is a float32 product, exact (|C| <= 2^19 with any grid, |S| <= 32) and issued faster than
+// v_mul_i32_i24.  The 8B gate/up and down at 512 tokens, us, IQ3_S 704 -> 680, IQ2_XXS 675 -> 654, IQ4_XS 660 -> 628, IQ3_XXS
+// (a launch) 265 -> 258; not where it measured slower: Q2_K 907 -> 945, IQ2_XS (a launch) 312 -> 322, IQ2_S 304 -> 312, IQ3_S's
+// 32-token tile at 16 tokens 143.5 -> 144.9; nor IQ1's, whose 8 C may pass 2^24 with a caller's grid.
+template <int TY, int NT> constexpr bool tile_float_scales() {
+  return TY == IQ2_XXS || TY == IQ3_XXS || TY == IQ4_XS || (TY == IQ3_S && NT > 32);
+}
 template <int TY> constexpr bool tile_sums16() { return has_minimums<TY>(); }
 // a second int8 tile: neg's 0 / 1 (signed grids) or IQ1's -(7 + 2 down) for each 8 weights
 template <int TY> constexpr bool tile_second() { return has_signs<TY>() || is_iq1<TY>(); }
@@ -872,7 +881,8 @@ __global__ __launch_bounds__(256) void gemm_sb(Job J) {
         const v4i_t Bm = *(const v4i_t *)(wm + mrow * SBT_PITCH + 32 * gg + 16 * kh);
         const v16i_t zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         const int32_t S0 = sbyte(Sw[c0 >> 2], c0 & 3), S1 = sbyte(Sw[c1 >> 2], c1 & 3);
-        int32_t G[16];
+        std::conditional_t<tile_float_scales<TY, NT>(), float, int32_t> G[16];
+        const float F0 = (float)S0;
         if (tile_split<TY>()) {
           const v4i_t z4 = {0, 0, 0, 0};
           v16i_t lo = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, kh == 0 ? Bm : z4, zero, 0, 0, 0);
@@ -907,7 +917,10 @@ __global__ __launch_bounds__(256) void gemm_sb(Job J) {
             for (int r = 0; r < 16; r++) C[r] = 8 * C[r] + Cc[r];
           }
 #pragma unroll
-          for (int r = 0; r < 16; r++) G[r] = TY == Q2_K ? C[r] : __mul24(S0, C[r]);
+          for (int r = 0; r < 16; r++) {
+            if constexpr (tile_float_scales<TY, NT>()) G[r] = fmul(F0, (float)C[r]);
+            else G[r] = TY == Q2_K ? C[r] : __mul24(S0, C[r]);
+          }
         }
         v16f_t Mf;  // M0 v0 + M1 v1 (the K types' minimums against the sums of 16), exact in float32: |.| < 2^18
         if (has_minimums<TY>()) {  // an outer product with K = 2: A the tokens' sums of chunks c0 (lanes 0..31) and
@@ -1170,7 +1183,7 @@ hipError_t launch_sb_row(float *out, const char *w, const uint8_t *tab, int32_t 
   return hipGetLastError();
 }
 
-// a prompt (kSbTileMin tokens or more) of one job through the tile
+// a prompt or a few tokens of one job through the tile
 hipError_t launch_sb_tile(const Job &j, hipStream_t s) {
   if (j.r1 <= j.r0 || j.count <= 0) return hipSuccess;
   switch (j.type) {

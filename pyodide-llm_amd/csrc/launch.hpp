@@ -85,9 +85,9 @@ hipError_t launch_sb(const Job *jobs, int32_t njobs, hipStream_t s);
 // whether launch_sb_ready takes them
 bool sb_ready_takes(const Job *jobs, int32_t njobs);
 hipError_t launch_sb_ready(const char *x, const Job *jobs, int32_t njobs, hipStream_t s);
-// a prompt of kSbTileMin tokens or more of one job (the sb kinds), on the matrix cores: every (row, token)
+// a prompt or a few tokens of one job (the sb kinds; abi.cpp says which) on the matrix cores: every (row, token)
 // launch_sb's number
-constexpr int kSbTileMin = 16;
+constexpr int kSbTileMin = 16;  // what hq_job_path reports as a tile
 constexpr int64_t kSbTileFrameMax = (int64_t)1 << 24;  // frame and sframe of a job the tile takes: 128 tokens' offsets fit in int32
 hipError_t launch_sb_tile(const Job &job, hipStream_t s);
 // a few tokens or a prompt of Q4_K (q4k.hip): whether a job is one that its tiles take, and the launch of up to kMaxJobs such jobs

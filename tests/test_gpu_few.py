@@ -49,7 +49,9 @@ def matrix(rng, oracle, kind, rows, n):
 CASES = [("matmul_q8r", n, t, 0) for n in (32, 96, 288, 512, 1056, 1664) for t in (5, 16, 17, 33, 48, 64, 96)] + \
         [("matmul_q6r", n, t, 0) for n in (32, 288, 512, 1664) for t in (5, 16, 33, 49, 64)] + \
         [(k, n, t, 4) for k in ("matmul_q8r", "matmul_q6r") for n in (32, 512, 1664) for t in (5, 33)] + \
-        [(k, n, t, 0) for k in ("matmul_t2r", "matmul_b1r") for n in (128, 384, 512, 1664) for t in (3, 16, 17, 33, 160, 400)]
+        [(k, n, t, 0) for k in ("matmul_t2r", "matmul_b1r") for n in (128, 384, 512, 1664) for t in (3, 16, 17, 33, 160, 400)] + \
+        [("matmul_q8r", 288, 130, 0), ("matmul_q8r", 512, 130, 4), ("matmul_q6r", 288, 130, 0),  # gemm.hip's tiles of several
+         ("matmul_t2r", 384, 420, 0), ("matmul_b1r", 384, 420, 0)]  # jobs in a launch, beyond the few-token tiles
 
 
 @pytest.mark.parametrize("kind,n,tokens,shift", CASES)

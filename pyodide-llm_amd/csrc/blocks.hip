@@ -1024,13 +1024,15 @@ hipError_t launch_tile_nt(const Job &j, int nrt, hipStream_t s) {
 }
 
 // the widest tile (128 for the tile_wide types, 64, 32 tokens) that still makes at least two blocks a compute unit:
-// a wider one decodes each block of weights for more tokens, a narrower one has more blocks to hide a block's waits
+// a wider one decodes each block of weights for more tokens, a narrower one has more blocks to hide a block's waits;
+// never one whose half would hold every token (the 27B gate/up of IQ3_S, us, the widest whatever the tokens / this: 16
+// tokens 275 / 103, 64 tokens 278 / 139; of Q2_K, 16 tokens 189 / 103)
 template <int TY>
 hipError_t launch_tile_type(const Job &j, hipStream_t s) {
   const int nrt = (j.r1 - j.r0 + SBT_R - 1) / SBT_R;
   const int64_t want = 2 * (int64_t)cu_count();
-  const int nt = tile_wide<TY>() && (int64_t)nrt * ((j.count + 127) / 128) >= want ? 128
-               : (int64_t)nrt * ((j.count + 63) / 64) >= want ? 64 : 32;
+  const int nt = tile_wide<TY>() && j.count > 64 && (int64_t)nrt * ((j.count + 127) / 128) >= want ? 128
+               : j.count > 32 && (int64_t)nrt * ((j.count + 63) / 64) >= want ? 64 : 32;
   if constexpr (tile_wide<TY>())
     if (nt == 128) return launch_tile_nt<TY, 128>(j, nrt, s);
   return nt == 64 ? launch_tile_nt<TY, 64>(j, nrt, s) : launch_tile_nt<TY, 32>(j, nrt, s);

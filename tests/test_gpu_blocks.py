@@ -375,10 +375,10 @@ def test_q4k_tiles(pkg, arena, oracle, setup, n, rows, tokens):
 
 
 @pytest.mark.parametrize("name,t", [("IQ2_XS", 17), ("IQ1_M", 29), ("Q2_K", 10), ("IQ4_XS", 23)])
-@pytest.mark.parametrize("rows,tokens", [(40, 8), (40, 9), (16400, 6)])
+@pytest.mark.parametrize("rows,tokens", [(40, 8), (40, 9), (16400, 6), (16400, 32), (16400, 33), (16400, 65)])
 def test_few_tokens_on_the_tile(pkg, arena, oracle, setup, name, t, rows, tokens):
     """both sides of the line between the token kernel and the tile below 16 tokens (n 512: 16400 rows are a large
-    matrix), every (row, token) the oracle's"""
+    matrix, whose tile is as wide as its tokens allow: 32, 64 or 128), every (row, token) the oracle's"""
     row, tab = setup
     n = 512
     area = arena.alloc(34992)

@@ -231,13 +231,38 @@ int32_t run_together(std::vector<hq::Job> &jobs, hq::Kind kind, Launch launch) {
   return HQ_OK;
 }
 
-// The blocks' jobs that take the matrix-core tile: what would be three launches or more of the token kernel (4 tokens
-// each), or two of them for a large matrix.  Measured (the 8B gate/up and down, us, token kernel / tile): IQ3_S at 5 tokens
-// 131 / 144, 6 tokens 158 / 144, 9 tokens 209 / 144, 15 tokens 336 / 144; a 1024-wide model's IQ2_XXS at 8 tokens 34 / 36, 9
-// tokens 48 / 37, 15 tokens 57 / 37.
-bool blocks_tile_takes(const hq::Job &j) {
-  const bool large = (int64_t)(j.r1 - j.r0) * j.n >= (int64_t)1 << 23;
-  return j.count >= (large ? 6 : 9) && blocks_tile_fits(j);
+// What the blocks' token kernel takes for jobs of one type and count, in us: a launch's start and, for every round of
+// 16 (row, slice of up to 4 tokens) a compute unit, a step per 1000 values of a row.  Fitted to 16 sets of row counts x 10
+// row lengths x 4 to 15 tokens x the ten types, each run both ways: the choice by it is within 0.2 % of the faster way on
+// average and never 15 % slower than the token kernel.
+double blocks_token_us(int64_t n, int64_t rows, int32_t jobs, int32_t count) {
+  static constexpr double kStart = 3.2, kStep[hq::kGemvMaxTokens + 1] = {0, 0.46, 0.88, 1.4, 2.06};
+  const int64_t round = 16 * (int64_t)hq::cu_count();
+  const auto launches = [&](int32_t tokens, int64_t slices) {
+    if (!slices || !tokens) return 0.0;
+    return kStart * (double)((jobs * slices + hq::kMaxJobs - 1) / hq::kMaxJobs) +
+           0.001 * kStep[tokens] * (double)n * (double)((rows * slices + round - 1) / round);
+  };
+  return launches(hq::kGemvMaxTokens, count / hq::kGemvMaxTokens) + launches(count % hq::kGemvMaxTokens, 1);
+}
+
+// The blocks' jobs below 16 tokens that take the matrix-core tile: those whose launches of the token kernel, with the phase's
+// other jobs of their type and count, would take longer.  A tile's blocks walk the row, so a matrix of few long rows leaves
+// most of the chip idle there.  Measured through hq_matmuls (IQ3_S, us, token kernel / tile): 14336 + 14336 rows of 4096 values
+// at 4 tokens 63 / 67, 5 tokens 81 / 67, 8 tokens 115 / 68; 4096 rows of 14336 at 8 tokens 66 / 78, 12 tokens 92 / 78; 2048
+// rows of 8192 at 8 tokens 23 / 46, 15 tokens 53 / 46.
+bool blocks_tile_takes(const hq::Job &j, const std::vector<hq::Job> &jobs) {
+  if (!blocks_tile_fits(j) || j.count < 4) return false;
+  if (j.count >= hq::kSbTileMin) return true;
+  double tiles = 0;
+  int64_t n = 0, rows = 0;
+  int32_t alike = 0;
+  for (const hq::Job &o : jobs) {
+    if (o.type != j.type || o.count != j.count || o.ws != j.ws || o.r1 == o.r0 || hq::q4k_tile(o)) continue;
+    tiles += hq::sb_tile_us(o);
+    n = std::max<int64_t>(n, o.n), rows += o.r1 - o.r0, alike++;
+  }
+  return tiles < blocks_token_us(n, rows, alike, j.count);
 }
 
 // runs jobs of one kind: few-token jobs and GEMV jobs (up to 4 tokens; more in slices of 4) and prompt tiles,
@@ -253,7 +278,7 @@ int32_t run_blocks(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t 
       continue;
     }
     // a prompt: the matrix-core tile (its offsets within a tile of tokens are 32-bit: frames under 16 MB)
-    if (blocks_tile_takes(j)) {
+    if (blocks_tile_takes(j, jobs)) {
       const int32_t st = hip_status(hq::launch_sb_tile(j, s), kind_name(kind));
       if (st) return st;
       continue;

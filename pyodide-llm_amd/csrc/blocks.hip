@@ -1185,6 +1185,26 @@ hipError_t launch_sb_row(float *out, const char *w, const uint8_t *tab, int32_t 
   return hipGetLastError();
 }
 
+// a tile of 32 tokens, measured with a block of it on a compute unit: us per 1000 values of a row; each further block on the
+// unit adds about half as much
+double sb_tile_us(const Job &j) {
+  const int64_t blocks = (j.r1 - j.r0 + SBT_R - 1) / SBT_R, cus = cu_count();
+  const auto step = [&] {
+    switch (j.type) {
+    case Q2_K: return 5.5;
+    case Q4_K: return 6.9;
+    case IQ2_XXS: return 4.8;
+    case IQ2_XS: return 5.4;
+    case IQ2_S: case IQ3_XXS: return 5.25;
+    case IQ3_S: return 5.1;
+    case IQ1_S: return 4.85;
+    case IQ1_M: return 6.75;
+    default: return 4.6;  // IQ4_XS
+    }
+  };
+  return 0.5 + 0.001 * j.n * step() * (1.0 + 0.5 * (double)((blocks + cus - 1) / cus - 1));
+}
+
 // a prompt or a few tokens of one job through the tile
 hipError_t launch_sb_tile(const Job &j, hipStream_t s) {
   if (j.r1 <= j.r0 || j.count <= 0) return hipSuccess;

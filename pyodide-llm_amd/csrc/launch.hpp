@@ -87,9 +87,10 @@ bool sb_ready_takes(const Job *jobs, int32_t njobs);
 hipError_t launch_sb_ready(const char *x, const Job *jobs, int32_t njobs, hipStream_t s);
 // a prompt or a few tokens of one job (the sb kinds; abi.cpp says which) on the matrix cores: every (row, token)
 // launch_sb's number
-constexpr int kSbTileMin = 16;  // what hq_job_path reports as a tile
+constexpr int kSbTileMin = 16;  // as many tokens always take it
 constexpr int64_t kSbTileFrameMax = (int64_t)1 << 24;  // frame and sframe of a job the tile takes: 128 tokens' offsets fit in int32
 hipError_t launch_sb_tile(const Job &job, hipStream_t s);
+double sb_tile_us(const Job &job);  // what that takes for 32 tokens or fewer, in us
 // a few tokens or a prompt of Q4_K (q4k.hip): whether a job is one that its tiles take, and the launch of up to kMaxJobs such jobs
 // of one token count
 bool q4k_tile(const Job &j);

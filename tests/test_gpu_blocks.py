@@ -375,12 +375,13 @@ def test_q4k_tiles(pkg, arena, oracle, setup, n, rows, tokens):
 
 
 @pytest.mark.parametrize("name,t", [("IQ2_XS", 17), ("IQ1_M", 29), ("Q2_K", 10), ("IQ4_XS", 23)])
-@pytest.mark.parametrize("rows,tokens", [(40, 8), (40, 9), (16400, 6), (16400, 32), (16400, 33), (16400, 65)])
-def test_few_tokens_on_the_tile(pkg, arena, oracle, setup, name, t, rows, tokens):
-    """both sides of the line between the token kernel and the tile below 16 tokens (n 512: 16400 rows are a large
-    matrix, whose tile is as wide as its tokens allow: 32, 64 or 128), every (row, token) the oracle's"""
+@pytest.mark.parametrize("n,rows,tokens", [(512, 40, 3), (512, 40, 4), (512, 40, 9), (2048, 40, 4), (2048, 40, 8), (2048, 40, 15),
+                                           (512, 16400, 4), (512, 16400, 6), (512, 16400, 32), (512, 16400, 33),
+                                           (512, 16400, 65)])
+def test_few_tokens_on_the_tile(pkg, arena, oracle, setup, name, t, n, rows, tokens):
+    """both sides of the line between the token kernel and the tile below 16 tokens (a short row's 4 tokens, a long row's 15),
+    and a large matrix, whose tile is as wide as its tokens allow (32, 64 or 128), every (row, token) the oracle's"""
     row, tab = setup
-    n = 512
     area = arena.alloc(34992)
     L = pkg.library()
     assert L.hq_sb_tables_ex(area, arena.put(row), None) == 0

@@ -236,7 +236,7 @@ int32_t run_together(std::vector<hq::Job> &jobs, hq::Kind kind, Launch launch) {
 // row lengths x 4 to 15 tokens x the ten types, each run both ways: the choice by it is within 0.2 % of the faster way on
 // average and never 15 % slower than the token kernel.
 double blocks_token_us(int64_t n, int64_t rows, int32_t jobs, int32_t count) {
-  static constexpr double kStart = 3.2, kStep[hq::kGemvMaxTokens + 1] = {0, 0.46, 0.88, 1.4, 2.06};
+  static constexpr double kStart = 3.2, kStep[hq::kGemvMaxTokens + 1] = {0, 0.46, 0.88, 1.5, 2.06};
   const int64_t round = 16 * (int64_t)hq::cu_count();
   const auto launches = [&](int32_t tokens, int64_t slices) {
     if (!slices || !tokens) return 0.0;
@@ -265,6 +265,20 @@ bool blocks_tile_takes(const hq::Job &j, const std::vector<hq::Job> &jobs) {
   return tiles < blocks_token_us(n, rows, alike, j.count);
 }
 
+// Q4_K's jobs below 16 tokens that take its own tiles (q4k.hip), by the same comparison.  Measured (us, token kernel / tile): 4096
+// rows of 14336 values at 3 tokens 33 / 43, 4 tokens 41 / 43, 5 tokens 51 / 43; 2048 rows of 8192 at 4 tokens 24 / 26, 8
+// tokens 24 / 26, 9 tokens 32 / 26; 14336 + 14336 rows of 4096 at 3 tokens 54 / 28.
+bool q4k_takes(const hq::Job &j, const std::vector<hq::Job> &jobs) {
+  if (j.count >= hq::kSbTileMin) return true;
+  int64_t n = 0, rows = 0, blocks = 0;
+  int32_t alike = 0;
+  for (const hq::Job &o : jobs) {
+    if (o.count != j.count || o.r1 == o.r0 || !hq::q4k_tile(o)) continue;
+    n = std::max<int64_t>(n, o.n), rows += o.r1 - o.r0, blocks += (o.r1 - o.r0 + 15) / 16, alike++;
+  }
+  return hq::q4k_us(n, blocks) < blocks_token_us(n, rows, alike, j.count);
+}
+
 // runs jobs of one kind: few-token jobs and GEMV jobs (up to 4 tokens; more in slices of 4) and prompt tiles,
 // batched in launches of up to kMaxJobs
 int32_t run_blocks(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s) {
@@ -273,12 +287,13 @@ int32_t run_blocks(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t 
   std::vector<hq::Job> parts, q4k;
   for (const hq::Job &j : jobs) {
     if (j.r1 == j.r0 || j.count == 0) continue;
-    if (hq::q4k_tile(j)) {
+    const bool own = hq::q4k_tile(j);
+    if (own && q4k_takes(j, jobs)) {
       q4k.push_back(j);
       continue;
     }
     // a prompt: the matrix-core tile (its offsets within a tile of tokens are 32-bit: frames under 16 MB)
-    if (blocks_tile_takes(j, jobs)) {
+    if (!own && blocks_tile_takes(j, jobs)) {
       const int32_t st = hip_status(hq::launch_sb_tile(j, s), kind_name(kind));
       if (st) return st;
       continue;

@@ -91,9 +91,11 @@ constexpr int kSbTileMin = 16;  // as many tokens always take it
 constexpr int64_t kSbTileFrameMax = (int64_t)1 << 24;  // frame and sframe of a job the tile takes: 128 tokens' offsets fit in int32
 hipError_t launch_sb_tile(const Job &job, hipStream_t s);
 double sb_tile_us(const Job &job);  // what that takes for 32 tokens or fewer, in us
-// a few tokens or a prompt of Q4_K (q4k.hip): whether a job is one that its tiles take, and the launch of up to kMaxJobs such jobs
-// of one token count
+// a few tokens or a prompt of Q4_K (q4k.hip): whether a job is one that its tiles take (abi.cpp says which of them do below 16
+// tokens), what 16 tokens or fewer of `blocks` 16-row tiles of rows of n values take (us), and the launch of up to kMaxJobs such
+// jobs of one token count
 bool q4k_tile(const Job &j);
+double q4k_us(int64_t n, int64_t blocks);
 hipError_t launch_q4k(const Job *jobs, int32_t njobs, hipStream_t s);
 hipError_t launch_signed_dots(int32_t *out, const int8_t *a, const int8_t *b, hipStream_t s);
 

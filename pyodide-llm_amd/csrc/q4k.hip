@@ -261,6 +261,14 @@ bool q4k_tile(const Job &j) {
          j.frame < kSbTileFrameMax && j.sframe < kSbTileFrameMax && (int64_t)32 * (j.n >> 8) * kQ4kBytes < INT32_MAX;
 }
 
+// us per 1000 values of a row with one block of 16 rows x 16 tokens on a compute unit; another on it adds a fifth of that, and
+// past four (resident together) they take 0.8 each
+double q4k_us(int64_t n, int64_t blocks) {
+  const int64_t cus = cu_count(), each = (blocks + cus - 1) / cus;
+  const double some = 2.48 + 0.55 * (double)(each - 1), many = 0.8 * (double)each;
+  return 0.001 * (double)n * (some > many ? some : many);
+}
+
 // 16 x 16 tiles up to 32 tokens and for launches whose 32 x 32 tiles are fewer than one and a half a compute unit (a step
 // is a quarter as long, and four times the blocks share the chip: the 8B gate/up and down at 16 tokens 107 -> 67 us, at
 // 64 the down projection 64 -> 58, a 1024-wide model's at 64 28 -> 23); 32 x 32 otherwise (64 tokens of the 8B gate/up 87 ->

@@ -326,11 +326,13 @@ def test_signed_dots(k, arena):
 
 
 @pytest.mark.parametrize("n,rows,tokens", [(256, 33, 3), (512, 16, 16), (1280, 50, 17), (256, 1, 32), (1024, 65, 33),
+                                           (8192, 20, 8), (8192, 20, 9),
                                            (768, 12400, 33), (512, 12300, 70)])
 def test_q4k_tiles(pkg, arena, oracle, setup, n, rows, tokens):
     """Q4_K's own tiles (16-byte aligned blocks, three tokens or more): 16 x 16 tiles and, for launches of many tiles,
     32 x 32 ones, cut inside a tile, two jobs of one input in a launch, a row range inside the matrix, nothing else
-    written; and blocks 2 bytes into a word (the general tile or token kernel), the same numbers"""
+    written; long rows, whose 8 tokens take the token kernel and 9 the tiles; and blocks 2 bytes into a word (the general
+    tile or token kernel), the same numbers"""
     from pyodide_llm_amd import jobs
     row, tab = setup
     area = arena.alloc(34992)

@@ -134,3 +134,58 @@ def test_one_token_from_its_float32_input(pkg, arena, oracle, kind, n, place):
         assert same_bits(arena.get(out, F, r), want)
     assert np.array_equal(arena.get(acts, np.uint8, n), q.view(np.uint8))
     assert same_bits(arena.get(b, F, ng), scales)
+
+
+def special(rng, n):
+    """a token's input with groups of every size, zeros, a NaN and an infinity (in groups the outputs of which are then NaN)"""
+    return activations(rng, 1, max(n, 128))[0, :n] if n >= 128 else rng.standard_normal(n).astype(F)
+
+
+def alike(got, want):
+    """the same bits, any NaN as any other"""
+    nan = np.isnan(want)
+    return np.array_equal(np.isnan(got), nan) and same_bits(got[~nan], want[~nan])
+
+
+BLOCK_READY = [(t, n) for t in ("Q2_K", "Q4_K", "IQ2_XXS", "IQ2_XS", "IQ2_S", "IQ3_XXS", "IQ3_S", "IQ1_S", "IQ1_M", "IQ4_XS")
+               for n in (256, 4352, 8192, 8448)] + [("Q4_K", 1280), ("Q4_K", 14336), ("Q4_K", 14592)]
+
+
+@pytest.mark.parametrize("name,n", BLOCK_READY)
+@pytest.mark.parametrize("shift,form", [(0, "plain"), (2, "special"), (0, "over x")])
+def test_one_token_of_blocks_from_its_float32_input(pkg, arena, oracle, name, n, shift, form):
+    """the same for llama.cpp's blocks: rows of 16 and 64 lanes, one round and several of the block's quantization, blocks
+    that start on 16 bytes and not, on both sides of the width it is done to; the bytes, scales and sums left in a / b"""
+    import blocks_model as bm
+    from pyodide_llm_amd import jobs
+    t = jobs.BLOCK_TYPES[name][0]
+    rng = np.random.default_rng(n + t)
+    x = special(rng, n) if form == "special" else rng.standard_normal(n).astype(F)
+    rows = (37, 9)
+    acts = arena.alloc(2 * n, fill=np.full(2 * n, 0xAA, np.uint8))
+    ax = arena.put(np.concatenate([x, np.zeros(64, F)]))
+    outs = [arena.alloc(4 * r, fill=np.full(r, -7, F)) for r in rows]
+    if form == "over x":
+        outs = [ax, ax + 4 * rows[0]]
+    q, scales = oracle.quantize_x(x, 0)
+    area = oracle.sums_x(q.view(np.int8), scales)
+    row = bm.codebooks(rng)
+    tab, tables = oracle.sb_tables(row), arena.alloc(34992)
+    L = pkg.library()
+    assert L.hq_sb_tables_ex(tables, arena.put(row), None) == 0
+    table, wants = [], []
+    for r, out in zip(rows, outs):
+        w = bm.random_blocks(rng, t, r * (n // 256))
+        at = arena.alloc(w.size + 16) + shift
+        arena.write(at, w)
+        wants.append(oracle.matmul_sbr(q.view(np.int8), area, w, tab, n, t))
+        table.append(jobs.job("matmul_sbr", out, acts, acts + n, at, tables, t, n, rows=r))
+    assert jobs.matmuls(L, ax, 4 * n, table) == 0, L.hq_last_error_message()
+    for out, r, want in zip(outs, rows, wants):
+        assert alike(arena.get(out, F, r), want)
+    got = arena.get(acts, np.uint8, 2 * n)
+    left = np.ascontiguousarray(area).view(np.uint8)
+    assert np.array_equal(got[:n], q.view(np.uint8))
+    assert alike(got[n:n + n // 8].view(F), left[:n // 8].view(F))
+    assert np.array_equal(got[n + n // 8:n + left.size], left[n // 8:])
+    assert np.all(got[n + left.size:] == 0xAA)

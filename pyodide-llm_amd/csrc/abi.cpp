@@ -50,18 +50,24 @@ int32_t path_of(hq::Kind kind, const hq::Job &j) {
   return j.count >= kGemmMinTokens && hq::gemm_supported(kind) && tile_offsets_fit(kind, j);
 }
 
-// The jobs that few.hip's 16-token tiles take: from the token counts where its one pass over the weights beats the token
-// kernel's pass a 4 tokens, to those where gemm.hip's larger tiles fill the GPU: more for a small phase (`weights`: those of
-// the phase's jobs of one kind).  Measured both ways (us, token kernel or prompt tile / few.hip): an 8B layer of int8 at 4
-// tokens 65 / 76, 5 tokens 109 / 76, 48 tokens 141 / 138, 64 tokens 154 / 168, a 350M one (9.4 M weights of gate and up) at
-// 64 tokens 56 / 53, 96 tokens 59 / 54, 128 tokens 60 / 60; the 27B MLP of int6 at 4 tokens 70 / 90, 32 tokens 176 / 148, 48
-// tokens 179 / 187; ternary's at 2 tokens 37 / 66, 3 tokens 72 / 67, 160 tokens 333 / 318, 192 tokens 339 / 350, a 1B
-// ternary layer (33 M) at 256 tokens 176 / 140, a 350M one at 400 tokens 117 / 93.
-bool few_tokens(hq::Kind kind, const hq::Job &j, int64_t weights) {
+// The jobs that few.hip's 16-token tiles take: those whose launch, with the phase's other jobs of their count and wc-ness, would
+// take longer on the token kernel (below 16 tokens) or on the prompt tiles.  Their one pass over the weights beats the token kernel's
+// pass a 4 tokens unless the rows are long and few (a tile's blocks walk a row), and the larger tiles until those fill the GPU.
+// Fitted to 25 sets of row counts x 14 row lengths x these counts x each packing with and without wc, each run both ways: the choice
+// by them is within 0.5 % of the faster way on average, and never more than 22 % slower than the other path.  Measured (us, token
+// kernel or prompt tile / few.hip): int8, 14336 + 14336 rows of 4096 values, 5 tokens 50 / 35, 16 tokens 40 / 37, 24 tokens
+// 42 / 46; 2048 rows of 8192, 8 tokens 12.7 / 13.4, 9 tokens 17.9 / 13.5, 96 tokens 34 / 26; ternary, 2048 rows of 8192, 8
+// tokens 12 / 20, 13 tokens 22 / 20, 320 tokens 74 / 50; 8192 + 8192 rows of 2048, 160 tokens 53 / 47, 256 tokens 55 / 68.
+bool few_tokens(hq::Kind kind, const hq::Job &j, const std::vector<hq::Job> &jobs) {
   const bool signs = hq::signs_kind(kind);
-  const int32_t least = signs ? 3 : 5;
-  const int32_t most = signs ? (weights < (40 << 20) ? 400 : 160) : weights < (10 << 20) ? 96 : kind == hq::Q6R ? 40 : 48;
-  return hq::gemm_supported(kind) && j.count >= least && j.count <= most && tile_offsets_fit(kind, j);
+  if (j.count < (signs ? 3 : 5) || j.count > (signs ? 400 : 128)) return false;
+  if (!hq::gemm_supported(kind) || !tile_offsets_fit(kind, j)) return false;
+  std::vector<hq::Job> alike;
+  for (const hq::Job &o : jobs)
+    if (o.r1 > o.r0 && o.count == j.count && (o.wc != nullptr) == (j.wc != nullptr)) alike.push_back(o);
+  const int32_t m = (int32_t)alike.size();
+  const double other = j.count < kGemmMinTokens ? hq::gemv_us(kind, alike.data(), m) : hq::gemm_us(kind, alike.data(), m);
+  return hq::few_us(kind, alike.data(), m) < other;
 }
 
 int32_t fail(int32_t code, const char *fmt, ...) {
@@ -328,11 +334,9 @@ int32_t run_jobs(hq::Kind kind, const std::vector<hq::Job> &jobs, hipStream_t s)
   if (hq::blocks_kind(kind)) return run_blocks(kind, jobs, s);
   std::vector<hq::Job> gemv[hq::kGemvMaxTokens + 1][2];  // by token count, by wc-ness
   std::vector<hq::Job> few, tiles;
-  int64_t weights = 0;
-  for (const hq::Job &j : jobs) weights += (int64_t)(j.r1 - j.r0) * j.n;
   for (const hq::Job &j : jobs) {
     if (j.r1 == j.r0 || j.count == 0) continue;
-    if (few_tokens(kind, j, weights)) {
+    if (few_tokens(kind, j, jobs)) {
       few.push_back(j);
       continue;
     }

@@ -487,6 +487,17 @@ hipError_t launch_few_tile(const Job *jobs, int32_t njobs, hipStream_t s) {
   return nt == 2 ? launch_few_of<Few<PACK, WC, WIDE, RT, 2>>(jobs, njobs, s) : launch_few_of<Few<PACK, WC, WIDE, RT, 1>>(jobs, njobs, s);
 }
 
+// Row steps of few tiles, measured: us per 1000 values of a row with 1, 2 (, 3) blocks of the tile on a compute unit, as many
+// as its LDS and registers let in, by token sub-tiles (further blocks wait their turn); and what a launch takes besides,
+// and for each block on a unit
+struct FewCost {
+  double start, block;
+  double step[4][3];
+};
+constexpr FewCost kFewInt8{4.5, 1.2, {{1.05, 1.95}, {1.9, 2.95}, {2.45, 3.8}, {3.05, 4.65}}};
+constexpr FewCost kFewInt6{4.5, 1.8, {{1.42, 1.92}, {2.6, 3.2, 4.6}, {3.15, 4.0}}};
+constexpr FewCost kFewSigns{2.5, 0.0, {{1.85, 2.4, 3.5}, {4.25, 5.05, 6.45}}};
+
 // every job's scales in 16-byte runs a step (Few's WIDE)
 bool few_wide(const Job *jobs, int32_t njobs) {
   uintptr_t bits = 0;
@@ -505,6 +516,22 @@ hipError_t launch_few_pack(const Job *jobs, int32_t njobs, hipStream_t s) {
 }
 
 }  // namespace
+
+double few_us(Kind kind, const Job *jobs, int32_t njobs) {
+  const bool signs = signs_kind(kind);
+  const int pack = signs ? 2 : kind == Q8R ? 8 : 6, rt = few_rows(pack), most = few_most(pack);
+  const int subs = (jobs[0].count + 15) / 16, tiles = (subs + most - 1) / most, nt = (subs + tiles - 1) / tiles;
+  int64_t blocks = 0, n = 0;
+  for (int j = 0; j < njobs; j++) {
+    blocks += (int64_t)((jobs[j].r1 - jobs[j].r0 + 16 * rt - 1) / (16 * rt)) * tiles;
+    if (jobs[j].n > n) n = jobs[j].n;
+  }
+  const FewCost &c = signs ? kFewSigns : pack == 8 ? kFewInt8 : kFewInt6;
+  const double *step = c.step[nt - 1];
+  const int64_t each = (blocks + cu_count() - 1) / cu_count(), in = step[2] > 0 ? 3 : 2;
+  return c.start + c.block * (double)each +
+         0.001 * (double)n * ((double)(each / in) * step[in - 1] + (each % in ? step[each % in - 1] : 0.0));
+}
 
 hipError_t launch_few(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s) {
   if (njobs < 1 || njobs > kMaxJobs) return hipErrorInvalidValue;

@@ -975,6 +975,25 @@ bool short_tiles(const Job *jobs, int32_t njobs, int token_tiles) {
 
 bool gemm_supported(Kind kind) { return kind == Q8R || kind == Q6R || signs_kind(kind); }
 
+// The tiles on a compute unit times what each takes per 1000 values of a row, measured: 32-row tiles of int8 / int6 (up to three
+// a unit, one round), 64-row ones (two a unit), ternary's and binary's (one; a 96-row one 0.87 of a 128-row one)
+double gemm_us(Kind kind, const Job *jobs, int32_t njobs) {
+  const int tt = (jobs[0].count + BT - 1) / BT;
+  const int64_t cus = cu_count();
+  int64_t n = 0;
+  for (int j = 0; j < njobs; j++)
+    if (jobs[j].n > n) n = jobs[j].n;
+  const auto each = [&](int rows) { return (double)((tiles_of(jobs, njobs, rows, tt) + cus - 1) / cus); };
+  if (signs_kind(kind)) {
+    const bool low = ternary_rows(jobs, njobs, tt) == 96;
+    return 4.0 + 0.001 * (double)n * (13.2 * (low ? 0.87 * each(96) : each(128)) - 1.2);
+  }
+  const bool wc = jobs[0].wc != nullptr, q8 = kind == Q8R;
+  const double values = 0.001 * (double)n * (wc ? q8 ? 1.24 : 1.12 : 1.0);
+  if (short_tiles(jobs, njobs, tt)) return (q8 ? 7.7 : 9.0) + (q8 ? 3.05 : 3.55) * values * each(32);
+  return (q8 ? 3.9 : 8.0) + ((q8 ? 4.55 : 5.1) * values + (q8 ? 3.9 : 3.7)) * each(64);
+}
+
 hipError_t launch_gemm(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s) {
   if (njobs < 1 || njobs > kMaxJobs) return hipErrorInvalidValue;
   const int tt = (jobs[0].count + BT - 1) / BT;

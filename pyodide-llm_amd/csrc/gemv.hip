@@ -1280,6 +1280,46 @@ hipError_t launch_gemv_ready(Kind kind, const char *x, const Job *jobs, int32_t 
   return hipGetLastError();
 }
 
+// Slices of up to four tokens, kMaxJobs a launch, the rest of the tokens a launch after.  Measured: a launch's start, then a
+// token's step per 1000 values of a row for every round of blocks over the compute units (a round of 16-lane int8 / int6 rows, twice
+// as many, counts twice), ternary's and binary's by the lanes of a row and by what of the tokens' staged bytes a unit's LDS holds;
+// int8 and int6 no less than the weights' bytes and the rows take, read a slice.
+double gemv_us(Kind kind, const Job *jobs, int32_t njobs) {
+  const bool signs = signs_kind(kind), q8 = kind == Q8R, bin = binary_kind(kind);
+  int nmax = 0;
+  int64_t rows = 0;
+  double bytes = 0;
+  for (int j = 0; j < njobs; j++) {
+    nmax = std::max(nmax, jobs[j].n);
+    rows += jobs[j].r1 - jobs[j].r0;
+    bytes += (double)(jobs[j].r1 - jobs[j].r0) * jobs[j].n * ((q8 ? 1.125 : 0.875) + (jobs[j].wc ? 0.125 : 0.0));
+  }
+  const auto launches = [&](int T, int slices) {
+    if (!T || !slices) return 0.0;
+    const double many = (double)((njobs * slices + kMaxJobs - 1) / kMaxJobs), values = 0.001 * nmax * T;
+    const auto rounds = [&](int rpb) {
+      const int64_t cus = cu_count();
+      return std::max(many, (double)((slices * blocks_of(jobs, njobs, rpb) + cus - 1) / cus));
+    };
+    if (!signs) {
+      const int lanes = relaxed_lanes(kind, T, nmax);
+      const double each = T == 1 ? rounds(16) : rounds(relaxed_threads(T, true) / lanes) * (lanes == 16 ? 2 : 1);
+      const double row = 1e-4 * (T == 1 ? (q8 ? 1.9 : 2.4) : (q8 ? 0.76 : 1.5));
+      const double read = slices * (1e-6 * (q8 ? 0.144 : 0.125) * bytes + row * (double)rows);
+      return (q8 ? 5.5 : 4.4) * many + std::max((q8 ? 0.134 : 0.2) * values * each, read);
+    }
+    const int lanes = ternary_lanes(nmax);
+    const size_t staged = ternary_stage_bytes(T, nmax);
+    const double step = staged > kTernaryStageMax           ? (bin ? 0.281 : 0.293)
+                        : lanes == 8                        ? (bin ? 0.357 : 0.27)
+                        : lanes == 16                       ? (bin ? 0.357 : 0.186)
+                        : 3 * staged <= (size_t)160 * 1024 ? (bin ? 0.143 : 0.108)
+                                                           : (bin ? 0.2 : 0.174);
+    return (bin ? 5.0 : 3.8) * many + step * values * rounds(256 / lanes);
+  };
+  return launches(kGemvMaxTokens, jobs[0].count / kGemvMaxTokens) + launches(jobs[0].count % kGemvMaxTokens, 1);
+}
+
 // jobs: one kind, one token count (1..4), one wc-ness (all with corrections or all without)
 hipError_t launch_gemv(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s) {
   return launch_batch(kind, jobs, njobs, s);

@@ -121,6 +121,12 @@ hipError_t launch_gemm(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s)
 // none, up to kMaxJobs a launch
 hipError_t launch_few(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s);
 
+// What jobs of one kind, token count and wc-ness (any number of them and of tokens) take on each of the three paths, in us from the
+// same base: estimates by which a launch's path is chosen (few_tokens in abi.cpp)
+double gemv_us(Kind kind, const Job *jobs, int32_t njobs);
+double few_us(Kind kind, const Job *jobs, int32_t njobs);
+double gemm_us(Kind kind, const Job *jobs, int32_t njobs);
+
 // the relaxed int8 prompt tile to float32 tolerance (gemm_tol.hip): the job's activations widened into `work`
 // (tol_work_bytes(n, count) bytes, 256-byte aligned), then the tiles; job.wc is not read (corrections derived)
 int64_t tol_work_bytes(int32_t n, int32_t count);

@@ -1,6 +1,6 @@
 """A few tokens on the matrix cores (few.hip), as hq_phase runs them: every (row, token) bit for bit the oracle's token
 kernel, at the edges of its tiles (16 rows, 32 of ternary and binary; 16 to 64 tokens), of its stages (256 or 512 values
-of a row), of its rule (the fewest and most tokens it takes), with groups past the fours, with scales that allow no
+of a row), of its rule (the fewest and most tokens it takes, few long rows), with groups past the fours, with scales that allow no
 16-byte loads, jobs of several row counts and both correction forms in one call, and no word outside the outputs
 written."""
 import numpy as np
@@ -50,8 +50,11 @@ CASES = [("matmul_q8r", n, t, 0) for n in (32, 96, 288, 512, 1056, 1664) for t i
         [("matmul_q6r", n, t, 0) for n in (32, 288, 512, 1664) for t in (5, 16, 33, 49, 64)] + \
         [(k, n, t, 4) for k in ("matmul_q8r", "matmul_q6r") for n in (32, 512, 1664) for t in (5, 33)] + \
         [(k, n, t, 0) for k in ("matmul_t2r", "matmul_b1r") for n in (128, 384, 512, 1664) for t in (3, 16, 17, 33, 160, 400)] + \
-        [("matmul_q8r", 288, 130, 0), ("matmul_q8r", 512, 130, 4), ("matmul_q6r", 288, 130, 0),  # gemm.hip's tiles of several
-         ("matmul_t2r", 384, 420, 0), ("matmul_b1r", 384, 420, 0)]  # jobs in a launch, beyond the few-token tiles
+        [("matmul_q8r", 288, 130, 0), ("matmul_q8r", 512, 130, 4), ("matmul_q6r", 288, 130, 0),  # gemm.hip's tiles of several jobs
+         ("matmul_t2r", 384, 420, 0), ("matmul_b1r", 384, 420, 0)] + \
+        [("matmul_q8r", 512, 128, 0), ("matmul_q6r", 512, 128, 0)] + \
+        [(k, 16384, t, 0) for k in ("matmul_q8r", "matmul_q6r", "matmul_t2r", "matmul_b1r") for t in (7, 8)]  # few long rows: 8
+#                                       tokens are cheaper in one launch of the token kernel, 7 (two launches) on the tiles
 
 
 @pytest.mark.parametrize("kind,n,tokens,shift", CASES)

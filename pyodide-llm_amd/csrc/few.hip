@@ -57,19 +57,26 @@ HQ_DEV rsrc4 few_resource(const char *base, int64_t bytes) {
   r[3] = 0x00020000;
   return r;
 }
-// lane l's SIZE bytes at r + vo + so land at LDS address dst + max(SIZE, 4) l (2 bytes zero-extended); past r's size: 0
+// Lane l's SIZE bytes at r + vo + so land at LDS address dst + max(SIZE, 4) l (2 bytes zero-extended); past r's size: 0.
+// M0, which the loads take their LDS address from, is declared as written (a reserved register: the compiler warns that it
+// does not allocate it).  A vector memory instruction may read a scalar register five wait states after a vector
+// instruction (v_readfirstlane) wrote it, and the compiler, which would insert these, does not look into the assembly:
+// FewLoads::settle() waits them once, and what the loads read later comes from scalar instructions.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 template <int SIZE>
 HQ_DEV void dma(rsrc4 r, uint32_t dst, uint32_t vo, uint32_t so) {
   if (SIZE == 16)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(dst), "v"(vo), "s"(r), "s"(so) : "memory");
+                 :: "s"(dst), "v"(vo), "s"(r), "s"(so) : "m0", "memory");
   else if (SIZE == 4)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-                 :: "s"(dst), "v"(vo), "s"(r), "s"(so) : "memory");
+                 :: "s"(dst), "v"(vo), "s"(r), "s"(so) : "m0", "memory");
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_ushort %1, %2, %3 offen lds"
-                 :: "s"(dst), "v"(vo), "s"(r), "s"(so) : "memory");
+                 :: "s"(dst), "v"(vo), "s"(r), "s"(so) : "m0", "memory");
 }
+#pragma clang diagnostic pop
 
 // ---- a stage's layout ------------------------------------------------------------------------------------------------
 // PACK: bits of a weight as stored (8 int8, 6 int6, 2 ternary, 1 binary).  WIDE: the int8 / int6 rows' and every token's
@@ -196,6 +203,12 @@ struct FewLoads {
           off[i] = scales(at, L::SLANE, (uint32_t)sb);
         }
       });
+  }
+
+  // the resources and the wave's number are in scalar registers, and a load may read them (dma)
+  HQ_DEV void settle() const {
+    asm volatile("s_nop 4" :: "s"(wave), "s"(rw), "s"(rx), "s"(rs), "s"(rxs));
+    if (L::WC) asm volatile("s_nop 4" :: "s"(rc));
   }
 
   // the wave's loads of a stage into the stage buffer at `base`; past the last stage they read nothing (sizes and
@@ -370,6 +383,7 @@ __global__ __launch_bounds__(kFewThreads, 2) void gemm_few(FewBatch batch) {
 
   const uint32_t lds0 = lds_addr(lds);
   const FewLoads<L> loads(J, row0, tok0, k);
+  loads.settle();
 #pragma unroll
   for (int s = 0; s < L::RING - 1; s++) loads.load(lds0 + s * L::STAGE, s, stages);
   float acc[RT][NT][4], last[RT][NT][4];  // the chain's sums; the term of the group past the fours (chains k < tail)

@@ -282,11 +282,13 @@ int32_t hq_matmul_q8r_tile_tol_ex(void *xout, const void *xq, const void *xs, co
  * reference: none. */
 int32_t hq_tol_min_tiles(int32_t tiles);
 
-/* Which kernels take a job of `kind` (hq_phase's numbers), row length n and `count` tokens whose activations are
- * frame bytes apart and their scales sframe: 1 the matrix-core tile (16 tokens or more, and every offset within a
- * tile of 64 tokens, 128 for llama.cpp's blocks, and of 128 rows below 4 GiB), 0 the token kernel (4 tokens a
- * launch: the same numbers), -1 a kind not run here.  (The counts between, about 5 to 64 tokens, run on the matrix
- * cores' few-token tiles whichever of the two this says: the same numbers.)  Host-only: no device is touched. */
+/* Whether the matrix cores' prompt tiles can take a job of `kind` (hq_phase's numbers), row length n and `count` tokens whose
+ * activations are frame bytes apart and their scales sframe: 1 they can (16 tokens or more, and every offset within a
+ * tile of 64 tokens, 128 for llama.cpp's blocks, and of 128 rows below 4 GiB), 0 they cannot, -1 a kind not run here.
+ * It is not the choice of a launch's kernels, which also goes by its rows, row lengths and tokens: where the offsets fit, tiles
+ * of 16 tokens take int8 and int6 from 5 to 128 tokens and ternary and binary from 3 to 400, and the blocks' tiles take
+ * theirs from 3 (Q4_K whose blocks start on 16 bytes) or 4, where they are estimated to be faster than the token kernel (4
+ * tokens a launch) or the prompt tiles.  Every path gives the same numbers.  Host-only: no device is touched. */
 int32_t hq_job_path(int32_t kind, int32_t n, int32_t count, int64_t frame, int64_t sframe);
 
 /* The ceilings the kernels are measured against (no counterpart on this path: the reference's CPU ceiling loops,

@@ -39,10 +39,9 @@ bool blocks_tile_fits(const hq::Job &j) {
   return j.frame > 0 && j.sframe > 0 && j.frame < hq::kSbTileFrameMax && j.sframe < hq::kSbTileFrameMax;
 }
 
-// Which kernels take a job: 1 the matrix-core tile, 0 the token kernel (4 tokens a launch).  The tiles keep a lane's
-// offsets within a tile in 32 bits: 64 tokens of activations (frame and sframe bytes apart: 128 for the blocks' tile)
-// and 128 rows of weights, so a job whose tile would reach 4 GiB from its first byte takes the token kernel, whose
-// addresses are 64-bit.
+// Whether the prompt tiles can take a job (hq_job_path).  The tiles keep a lane's offsets within a tile in 32 bits: 64 tokens
+// of activations (frame and sframe bytes apart: 128 for the blocks' tile) and 128 rows of weights, so a job whose tile would
+// reach 4 GiB from its first byte takes the token kernel, whose addresses are 64-bit.
 int32_t path_of(hq::Kind kind, const hq::Job &j) {
   if (hq::blocks_kind(kind)) {
     return j.count >= hq::kSbTileMin && blocks_tile_fits(j);

@@ -159,7 +159,7 @@ def test_job_path_keeps_tile_offsets_in_32_bits(pkg):
     n = 4096
     frame = n + n // 8
     assert L.hq_job_path(q8r, n, 2048, frame, frame) == 1
-    assert L.hq_job_path(q8r, n, 15, frame, frame) == 0  # under 16 tokens: the token kernel
+    assert L.hq_job_path(q8r, n, 15, frame, frame) == 0  # under 16 tokens: no prompt tile
     assert L.hq_job_path(q8, n, 2048, frame, frame) == 0  # no matrix-core tile for the plain form
     big = 1 << 26  # 64 tokens x 64 MiB reach 4 GiB
     assert L.hq_job_path(q8r, n, 2048, big - 4096, big - 4096) == 1

@@ -376,6 +376,45 @@ def test_q4k_tiles(pkg, arena, oracle, setup, n, rows, tokens):
         assert np.all(got[:, :5] == -7) and np.all(got[:, rows - 3:] == -7) and same_bits(got[-1, 5:rows - 3], want[5:rows - 3])
 
 
+@pytest.mark.parametrize("n,rows,tokens", [(768, 37, 3), (768, 37, 17), (512, 12300, 70)])
+def test_q4k_tiles_of_infinite_and_nan_scales(pkg, arena, oracle, setup, n, rows, tokens):
+    """activations' scales that are infinite or NaN, in both tiles: the same tokens as in the oracle and no others; and blocks
+    whose scale or minimum has a float16's largest exponent, which is a value like the others (65536 and more)"""
+    from pyodide_llm_amd import jobs
+    row, tab = setup
+    area = arena.alloc(34992)
+    L = pkg.library()
+    assert L.hq_sb_tables_ex(area, arena.put(row), None) == 0
+    rng = np.random.default_rng(n + rows + tokens)
+    frame = 2 * n
+    buf = np.zeros((tokens, frame), np.uint8)
+    ready = []
+    for t in range(tokens):
+        q, area_t = token_area(oracle, rng, n, 1.0 + t)
+        if t in (1, 2):
+            area_t = np.ascontiguousarray(area_t).copy()
+            area_t.view(np.uint8)[4 * t:4 * t + 4].view(F)[0] = np.inf if t == 1 else np.nan
+        buf[t, :n], buf[t, n:n + area_t.nbytes] = q.view(np.uint8), area_t.view(np.uint8)
+        ready.append((q, area_t))
+    blocks = bm.random_blocks(rng, 12, rows * (n // 256))
+    halves = blocks.reshape(rows, n // 256, 144)[:, :, :4].copy().view(np.float16)  # a block's scale and minimum
+    halves[1::4, 0, 0], halves[2::4, -1, 1], halves[3::8, 0, 0] = np.inf, np.inf, np.nan
+    blocks = blocks.reshape(rows, n // 256, 144).copy()
+    blocks[:, :, :4] = halves.view(np.uint8)
+    blocks = blocks.reshape(-1)
+    out = arena.alloc(4 * rows * tokens, fill=np.full(rows * tokens, -7, F))
+    a = arena.put(buf)
+    table = [jobs.job("matmul_sbr", out, a, a + n, arena.put(blocks), area, 12, n, rows=rows, count=tokens, os=4 * rows,
+                      as_=frame, bs=frame)]
+    assert jobs.phase(L, table) == 0, L.hq_last_error_message()
+    got = arena.get(out, F, rows * tokens).reshape(tokens, rows)
+    for t in sorted({0, 1, 2, tokens - 1}):
+        want = oracle.matmul_sbr(*ready[t], blocks, tab, n, 12)
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(got[t]), nan) and same_bits(got[t][~nan], want[~nan]), t
+        assert np.isfinite(want).all() == (t not in (1, 2))
+
+
 @pytest.mark.parametrize("name,t", [("IQ2_XS", 17), ("IQ1_M", 29), ("Q2_K", 10), ("IQ4_XS", 23)])
 @pytest.mark.parametrize("n,rows,tokens", [(512, 40, 3), (512, 40, 4), (512, 40, 9), (2048, 40, 4), (2048, 40, 8), (2048, 40, 15),
                                            (512, 16400, 4), (512, 16400, 6), (512, 16400, 32), (512, 16400, 33),

@@ -241,9 +241,10 @@ def tile_inputs(oracle, rng, n, count, frame, rows):
     return q
 
 
-@pytest.mark.parametrize("count", [1, 2, 3, 4, 5, 7, 8, 9, 16, 17, 33, 64, 65, 100])
+@pytest.mark.parametrize("count", [1, 2, 3, 4, 5, 7, 8, 9, 16, 17, 33, 64, 65, 100, 129])
 @pytest.mark.parametrize("ng", [1, 3, 4, 9, 13, 80])
 def test_q8r_tile(k, arena, oracle, count, ng):
+    """every path: the token kernel (four tokens a launch), the few-token tiles (5 to 128) and the prompt tiles"""
     rng = np.random.default_rng(1000 * ng + count)
     n = 32 * ng
     rows = 70
@@ -426,12 +427,12 @@ def test_relaxed_bytes_past_seven_bits(k, arena):
             assert same_bits(got[t], want), f"token {t} wc {bool(wca)}: {first_difference(got[t], want)}"
 
 
-@pytest.mark.parametrize("count", [2, 4, 5, 16, 40])
+@pytest.mark.parametrize("count", [2, 4, 5, 16, 40, 129])
 @pytest.mark.parametrize("ng", [13, 16])
 def test_q6r_many_tokens(pkg, arena, oracle, count, ng):
     """matmul_q6r over a prompt (no tile in the reference: a call a token, jobs.ts:471-475) through hq_phase, with
-    the corrections given, moved and derived (wc = NULL); 13 groups a row (the prompt tile loads a stage's scales four
-    bytes a lane) and 16 (sixteen bytes a lane)"""
+    the corrections given, moved and derived (wc = NULL); 13 groups a row (the tiles load a stage's scales four
+    bytes a lane) and 16 (sixteen bytes a lane); the prompt tiles from 129 tokens whatever the rows"""
     from pyodide_llm_amd import jobs
     rng = np.random.default_rng(77 + count + 1000 * ng)
     rows = 90
@@ -593,9 +594,9 @@ def test_ternary_largest_sums(k, arena, oracle):
 
 
 @pytest.mark.parametrize("count,groups", [(c, g) for c in [1, 2, 3, 4, 5, 7, 8, 9, 16, 17, 64, 65, 100]
-                                          for g in [1, 3, 9]] + [(4, 136), (3, 136), (2, 40)])
+                                          for g in [1, 3, 9]] + [(4, 136), (3, 136), (2, 40), (401, 1), (401, 9)])
 def test_t2r_tile(k, arena, oracle, count, groups):
-    """(4, 136): four tokens of 17408 activations are more than the token kernel stages in LDS (read through the L1)"""
+    """the token kernel, the few-token tiles and, at 401 tokens, the prompt tiles; (4, 136): four tokens of 17408 activations are more than the token kernel stages in LDS (read through the L1)"""
     n, codes, halves, rng = ternary_case(groups, rows=70, seed=500 + count)
     rows = 70
     wbytes = pack_ternary(codes)
@@ -633,19 +634,20 @@ def ternary_tile_rows(rows, token_tiles, cus):
 @pytest.mark.parametrize("height", [96, 128])
 @pytest.mark.parametrize("packing", ["ternary", "binary"])
 def test_signs_tile_heights(pkg, k, arena, oracle, height, packing):
-    """The ternary / binary prompt tile at both heights: 96 rows (a launch of few tiles: 301 rows cut at 3 and 299, 131
-    tokens) and 128 (a launch of two full rounds of 128-row tiles, sized from the device's CU count: ~32 row tiles
-    of 1024 tokens, cut at 5 and 21 short of the end); 3 groups of 128, rows cut inside the tiles."""
+    """The ternary / binary prompt tile at both heights: 96 rows (a launch of few tiles: 301 rows cut at 3 and 299, 451
+    tokens: more than the few-token tiles take) and 128 (a launch of two full rounds of 128-row tiles, sized from the device's CU count: ~32 row tiles
+    of 1024 tokens, cut at 5 and 21 short of the end); rows cut inside the tiles, of 9 groups of 128 (the ring of four
+    stages twice round) and 3."""
     import torch
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     if height == 96:
-        rows, r0, r1, count = 301, 3, 299, 131
+        rows, r0, r1, count = 301, 3, 299, 451
     else:
         count = 1024
         rows = 128 * ((2 * cus) // 16) + 26
         r0, r1 = 5, rows - 21
     assert ternary_tile_rows(r1 - r0, -(-count // 64), cus) == height
-    groups = 3
+    groups = 9 if height == 96 else 3
     if packing == "ternary":
         n, codes, halves, rng = ternary_case(groups, rows=rows, seed=900 + height)
         wbytes = pack_ternary(codes)
@@ -735,9 +737,10 @@ def test_signs_block_waves(k, arena, oracle, rows, packing):
 
 
 @pytest.mark.parametrize("count,groups", [(c, g) for c in [1, 2, 3, 4, 5, 7, 8, 9, 16, 17, 64, 65, 100]
-                                          for g in [1, 3, 9]] + [(4, 136), (3, 136), (2, 40), (33, 136)])
+                                          for g in [1, 3, 9]] + [(4, 136), (3, 136), (2, 40), (33, 136), (401, 1), (401, 9)])
 def test_b1r_tile(k, arena, oracle, count, groups):
-    """every count of tokens (the token kernel up to 4 at a time, the MFMA tiles from 16), rows cut anywhere"""
+    """every path (the token kernel up to 4 tokens at a time, the few-token tiles, the prompt tiles at 401), rows cut
+    anywhere"""
     rows = 70
     n, bits, bw, halves, rng = binary_case(groups, rows=rows, seed=700 + count)
     wq, wsa = arena.put(bw), arena.put(halves)

@@ -189,3 +189,43 @@ def test_one_token_of_blocks_from_its_float32_input(pkg, arena, oracle, name, n,
     assert alike(got[n:n + n // 8].view(F), left[:n // 8].view(F))
     assert np.array_equal(got[n + n // 8:n + left.size], left[n // 8:])
     assert np.all(got[n + left.size:] == 0xAA)
+
+
+@pytest.mark.parametrize("kind", ["matmul_q8r", "matmul_q6r"])
+@pytest.mark.parametrize("n", [32, 96, 288, 512, 1536])
+@pytest.mark.parametrize("form", ["wc", "derived"])
+@pytest.mark.parametrize("values", ["plain", "special"])
+@pytest.mark.parametrize("pairs", ["one a and b", "one a, two b"])
+def test_one_token_of_int8_and_int6_from_its_float32_input(pkg, arena, oracle, kind, n, form, values, pairs):
+    """the same for int8 and int6, corrections given and derived, with groups past the fours, of rows whose input's groups
+    hold a NaN and an infinity; every job's a / b hold the readied activations after the call, also where two jobs of one a
+    have a b each (which takes the input apart)"""
+    from pyodide_llm_amd import jobs
+    rng = np.random.default_rng(n)
+    ng = n // 32
+    x = special(rng, n) if values == "special" else rng.standard_normal(n).astype(F)
+    q, scales = oracle.quantize_x(x, 64)
+    a = arena.alloc(n + 16, fill=np.full(n + 16, 0xAA, np.uint8))
+    bs = [arena.alloc(n // 8 + 16, fill=np.full(n // 8 + 16, 0xAA, np.uint8)) for _ in range(2)]
+    table, wants = [], []
+    for i, r in enumerate((37, 9)):
+        ws = (rng.standard_normal(r * ng) * 0.02).astype(F)
+        if kind == "matmul_q6r":
+            w = pack6((4 * rng.integers(-32, 32, r * n)).astype(np.int8))
+            wc, product = oracle.six_sums(w), oracle.matmul_q6r
+        else:
+            w = rng.integers(-128, 128, r * n).astype(np.int8)
+            wc, product = oracle.int8_sums(w), oracle.matmul_q8r
+        out = arena.alloc(4 * r, fill=np.full(r, -7, F))
+        b = bs[i] if pairs == "one a, two b" else bs[0]
+        table.append(jobs.job(kind, out, a, b, arena.put(w), arena.put(ws), arena.put(wc) if form == "wc" else 0, n, rows=r))
+        wants.append((out, r, product(q, scales, w, ws, wc, n)))
+    L = pkg.library()
+    assert jobs.matmuls(L, arena.put(np.concatenate([x, np.zeros(64, F)])), 4 * n, table) == 0, L.hq_last_error_message()
+    for out, r, want in wants:
+        assert alike(arena.get(out, F, r), want)
+    got = arena.get(a, np.uint8, n + 16)
+    assert np.array_equal(got[:n], q.view(np.uint8)) and np.all(got[n:] == 0xAA)
+    for b in bs[:2 if pairs == "one a, two b" else 1]:
+        got = arena.get(b, np.uint8, n // 8 + 16)
+        assert alike(got[:n // 8].view(F), scales) and np.all(got[n // 8:] == 0xAA)

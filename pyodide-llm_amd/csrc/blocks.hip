@@ -18,7 +18,7 @@
 // through fold.hpp's LDS fold, lane k adding part k of the step's blocks in order, as the ternary kernels do.
 // A few tokens go 4 at a time through the same kernel (blocks_tile_takes in abi.cpp draws the line); a prompt through
 // the matrix-core tile below (gemm_sb): every (row, token) the token kernel's number either way.  (Q4_K whose blocks start
-// on 16 bytes takes q4k.hip's tiles from three tokens: the same numbers.)
+// on 16 bytes takes q4k.hip's tiles, from three tokens where they are faster: the same numbers.)
 #include <type_traits>
 
 #include "common.hpp"

@@ -37,7 +37,9 @@ typedef int32_t v4i __attribute__((ext_vector_type(4)));
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-// the ring's LDS: more stages (78 KB, two blocks a CU) measured no faster for 16 tokens and 4-7 % slower for 17..32
+// The ring's LDS where three stages leave room in it (binary, and two token sub-tiles of ternary and of int6 without wc: 34 to 39
+// KB, four blocks a CU by LDS); the others' three stages take 42 to 72 KB, two or three blocks.  Rings of 78 KB measured no
+// faster for 16 tokens and 4-7 % slower for 17..32
 constexpr int kFewLds = 39 * 1024;
 struct FewBatch {
   Job job[kMaxJobs];

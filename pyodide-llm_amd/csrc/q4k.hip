@@ -14,8 +14,9 @@
 //
 // Measured (the 8B gate/up and down through hq_matmuls, us, before: 4 tokens a launch of the token kernel below 16
 // tokens, blocks.hip's tile from 16): 4 tokens 108 -> 63, 15 tokens 353 -> 64, 16 tokens 187 -> 64, 32 tokens 190 -> 85,
-// 64 tokens 254 -> 115, 333 tokens 911 -> 477, 512 tokens 1127 -> 672 (160 -> 268 TOPS).  Of that, S times the integer
-// as a float32 product instead of v_mul_i32_i24, which issues slower: 333 tokens 521 -> 477, 512 tokens 728 -> 672.
+// 64 tokens 254 -> 111, 333 tokens 916 -> 459, 512 tokens 1127 -> 644 (160 -> 280 TOPS), passes back to back (a few after an idle
+// second: 720 to 795).  Of that, S times the integer as a float32 product instead of v_mul_i32_i24, which issues slower: 333
+// tokens 521 -> 477, 512 tokens 728 -> 672 when it was brought in.
 // What bounds a prompt: those 16 operations, 563 of a SIMD's cycles a pair and 32 x 32 outputs, beside 64 of the matrix
 // cores' (which add on this part: 459 TOPS at 2.2 GHz), and per step of a wave ~60 operations of scales and operands.
 // A few tokens: the steps' latency, one after the other down a row (56 steps of the down projection, 0.6 us each).

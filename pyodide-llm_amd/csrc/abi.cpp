@@ -52,10 +52,10 @@ int32_t path_of(hq::Kind kind, const hq::Job &j) {
 // The jobs that few.hip's 16-token tiles take: those whose launch, with the phase's other jobs of their count and wc-ness, would
 // take longer on the token kernel (below 16 tokens) or on the prompt tiles.  Their one pass over the weights beats the token kernel's
 // pass a 4 tokens unless the rows are long and few (a tile's blocks walk a row), and the larger tiles until those fill the GPU.
-// Fitted to 25 sets of row counts x 14 row lengths x these counts x each packing with and without wc, each run both ways; taken where
-// the estimate is 5 % below the other path's.  Over 18000 random calls (1 to 3 matrices of 48 to 30000 rows, 256 to 20000 values,
-// weights past the caches) the choice is within 0.6 % of the faster way on average, and 0.8 % of the calls are more than 3 %
-// slower than on the other path, 26 % at most (without the 5 %: 0.4 %, 1.6 % of them, 72 %).  Measured (us, token
+// Fitted to 25 sets of row counts x 14 row lengths x these counts x each packing with and without wc, each run both ways; over 18000
+// random calls (1 to 3 matrices of 48 to 30000 rows, 256 to 20000 values, weights past the caches) the choice is within 0.4 % of
+// the faster way on average, and 1.4 % of the calls are more than 3 % slower than on the other path, 30 % at most.  (Taken only
+// where 5 % below instead: 0.8 % of the calls, but 0.6 % on average; a 4864-wide layer of 45 tokens 211 -> 221.)  Measured (us, token
 // kernel or prompt tile / few.hip): int8, 14336 + 14336 rows of 4096 values, 5 tokens 50 / 35, 16 tokens 40 / 37, 24 tokens
 // 42 / 46; 2048 rows of 8192, 8 tokens 12.7 / 13.4, 9 tokens 17.9 / 13.5, 96 tokens 34 / 26; ternary, 2048 rows of 8192, 8
 // tokens 12 / 20, 13 tokens 22 / 20, 320 tokens 74 / 50; 8192 + 8192 rows of 2048, 160 tokens 53 / 47, 256 tokens 55 / 68.
@@ -68,7 +68,7 @@ bool few_tokens(hq::Kind kind, const hq::Job &j, const std::vector<hq::Job> &job
     if (o.r1 > o.r0 && o.count == j.count && (o.wc != nullptr) == (j.wc != nullptr)) alike.push_back(o);
   const int32_t m = (int32_t)alike.size();
   const double other = j.count < kGemmMinTokens ? hq::gemv_us(kind, alike.data(), m) : hq::gemm_us(kind, alike.data(), m);
-  return hq::few_us(kind, alike.data(), m) < 0.95 * other;
+  return hq::few_us(kind, alike.data(), m) < other;
 }
 
 int32_t fail(int32_t code, const char *fmt, ...) {

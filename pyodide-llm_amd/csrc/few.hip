@@ -545,8 +545,11 @@ double few_us(Kind kind, const Job *jobs, int32_t njobs) {
   const FewCost &c = signs ? kFewSigns : pack == 8 ? kFewInt8 : kFewInt6;
   const double *step = c.step[nt - 1];
   const int64_t each = (blocks + cu_count() - 1) / cu_count(), in = step[2] > 0 ? 3 : 2;
-  return c.start + c.block * (double)each +
-         0.001 * (double)n * ((double)(each / in) * step[in - 1] + (each % in ? step[each % in - 1] : 0.0));
+  const double rest = c.block * (double)each +
+                      0.001 * (double)n * ((double)(each / in) * step[in - 1] + (each % in ? step[each % in - 1] : 0.0));
+  // (scales loaded 4 bytes a lane cost these tiles 9 % more, the prompt tiles nothing: int8 with wc, 17740 rows of 288 values at 76
+  // tokens 23 us here, 13 there; the token kernel's rows of such lengths are slower too)
+  return c.start + (!signs && jobs[0].count >= 16 && !few_wide(jobs, njobs) ? 1.09 : 1.0) * rest;
 }
 
 hipError_t launch_few(Kind kind, const Job *jobs, int32_t njobs, hipStream_t s) {
